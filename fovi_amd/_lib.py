@@ -14,12 +14,12 @@ import torch
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libfovi_hip.so")
 
-ABI_VERSION = 33
+ABI_VERSION = 34
 F32, BF16, F8E4M3 = 0, 1, 2
 NEAREST, BILINEAR = 0, 1
 PAD_ZEROS, PAD_BORDER = 0, 1
 ACT_NONE, ACT_RELU = 0, 1
-W_ROWS, W_MFMA = 0, 1
+W_ROWS, W_MFMA, W_IMG = 0, 1, 2
 POOL_MAX, POOL_AVG, POOL_SUM, POOL_GAUSSIAN = 0, 1, 2, 3
 
 _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16, torch.float8_e4m3fn: F8E4M3}
@@ -30,7 +30,8 @@ EXPORTED = ("fovi_abi_version", "fovi_last_error", "fovi_sampler_fwd", "fovi_knn
             "fovi_quantize_e4m3", "fovi_knnpool_fwd", "fovi_knnconv_slotsum", "fovi_knnconv_bwd_x",
             "fovi_knn_logpolar_candidates", "fovi_knn_select", "fovi_knn_euclid_candidates", "fovi_local_rf_slots", "fovi_knnconv_dw_workspace_bytes",
             "fovi_knnconv_dw", "fovi_knnpool_bwd", "fovi_knnconv_last_path",
-            "fovi_knnconv_fwd_noalloc", "fovi_knnconv_wide_tiles")
+            "fovi_knnconv_fwd_noalloc", "fovi_knnconv_wide_tiles", "fovi_knnconv_weight_img_elems",
+            "fovi_knnconv_pack_weight_img", "fovi_knnconv_img_tables")
 
 
 class SamplerArgs(C.Structure):
@@ -80,6 +81,9 @@ class KnnConvArgs(C.Structure):
         ("fc_comb", C.c_void_p), ("fc_comb_off", C.c_void_p), ("fc_pmax", C.c_int32), ("wide_tiles", C.c_int32),
         ("vm_idx", C.c_void_p), ("vm_ev", C.c_void_p), ("vm_off", C.c_void_p), ("vm_j0", C.c_void_p),
         ("vm_w", C.c_void_p), ("vm_nb", C.c_int32), ("vm_cb", C.c_int32),
+        ("img_ent", C.c_void_p), ("img_points", C.c_void_p), ("img_nact", C.c_void_p), ("img_flag", C.c_void_p),
+        ("img_groups", C.c_int64), ("img_pp", C.c_int32), ("img_ib", C.c_int32), ("img_cb", C.c_int32),
+        ("reserved8", C.c_int32),
     ]
 
 
@@ -217,6 +221,15 @@ def load(path: str = LIB_PATH):
     lib.fovi_knnconv_pack_weight_mfma.argtypes = [C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p,
                                                   C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p]
     lib.fovi_knnconv_pack_weight_mfma.restype = C.c_int
+    lib.fovi_knnconv_weight_img_elems.argtypes = [C.c_int64, C.c_int64, C.c_int64, C.c_int32]
+    lib.fovi_knnconv_weight_img_elems.restype = C.c_int64
+    lib.fovi_knnconv_pack_weight_img.argtypes = [C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p,
+                                                 C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
+    lib.fovi_knnconv_pack_weight_img.restype = C.c_int
+    lib.fovi_knnconv_img_tables.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p,
+                                            C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p,
+                                            C.c_void_p, C.POINTER(C.c_double)]
+    lib.fovi_knnconv_img_tables.restype = C.c_int64
     lib.fovi_quantize_e4m3.argtypes = [C.POINTER(QuantizeArgs), C.c_void_p]
     lib.fovi_quantize_e4m3.restype = C.c_int
     lib.fovi_knnpool_fwd.argtypes = [C.POINTER(KnnPoolArgs), C.c_void_p]

@@ -50,6 +50,9 @@ __all__ = [
     "register_with_reference",
 ]
 
+# Smallest batch of the image-row kernel.
+IMG_MIN_BATCH = 8
+
 _KCHUNK = 64  # reduction chunk of the MFMA kernel; packed weights are padded to it
 
 # Attributes of a sensor point set the kNN layers read (those of the reference's
@@ -171,6 +174,16 @@ class _KnnConvFn(torch.autograd.Function):
         dx, dw = layer._backward(x, weight, dy, ctx.needs_input_grad[0], ctx.needs_input_grad[2])
         db = dy.sum(dim=(0, 2)).to(torch.float32) if ctx.has_bias and ctx.needs_input_grad[3] else None
         return dx, None, dw, db, None
+
+
+class _ImageRows:
+    """What the image-row kernel keeps per layer: host copies of the CSR tables it builds its own
+    from, the point order, the device tables per group size (at most five), the mean slot unions
+    and the plans per batch size."""
+
+    def __init__(self, slot_ptr, nbr):
+        self.slot_ptr, self.nbr = slot_ptr.cpu(), nbr.cpu()
+        self.order, self.tables, self.unions, self.plans = None, {}, {}, {}
 
 
 class KNNConvLayer(nn.Module, KNNBaseLayer):
@@ -351,6 +364,7 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         # that spreads the heavy slots' collision sums over the stream
         self._direct_tables = tiles
         self._packed = {}
+        self._img = _ImageRows(slot_ptr, nbr_sorted)
         order = None
         if tiles is not None:
             order = T.stream_slot_order(T.slot_stream_units(tiles), ahead=T.wide_tiles_of(tiles))
@@ -384,6 +398,9 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         # 256-channel tiles, tables within LDS): weights in MFMA-fragment order for the
         # 256 x 256-tile kernel (False: the row-packed kernels)
         self.mfma_weights = True
+        # batches of at least IMG_MIN_BATCH: the image-row kernel, which visits only the slots a
+        # point uses (False: the kernels whose tiles are points of one image)
+        self.image_rows = True
 
     def set_few_channel_geometry(self, geometries=None, knn_indices=None, slots=None, n_in=None, n_ref=None,
                                  device=None):
@@ -516,8 +533,11 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         self.slot_order = None if order is None else [int(v) for v in order]
         self._slot_order_dev = None if order is None else torch.tensor(self.slot_order, dtype=torch.int32,
                                                                           device=dev)
-        self._packed.pop(("mfma", torch.bfloat16), None)
-        self._packed.pop(("mfma", torch.float8_e4m3fn), None)
+        for dt in (torch.bfloat16, torch.float8_e4m3fn, torch.float32):
+            self._packed.pop(("mfma", dt), None)
+            self._packed.pop(("image", dt), None)
+        if self._img is not None:
+            self._img.tables = {}
 
     def _packed_weight_mfma(self, dtype=torch.bfloat16):
         """Weight in MFMA-fragment order (``fovi_knnconv_pack_weight_mfma``) for the current slot
@@ -566,6 +586,138 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
                 and self.tile_src is not None and 0 < self._zero_row <= T.WIDE_MAX_ROWS
                 and self._k <= 255 and x.stride(1) == 1 and x.stride(2) % align == 0
                 and x.stride(0) % align == 0 and x.data_ptr() % 16 == 0)
+
+    # -- image-row kernel ------------------------------------------------------
+    # (class defaults: a layer unpickled from a file without these attributes runs the other kernels)
+    image_rows = False
+    _img = None
+
+    def _image_plan(self, batch):
+        """``(work, (rows per workgroup / 32, images per point, 32-column blocks per wave))`` of the
+        image-row kernel for ``batch`` images: the least estimated work, in slots visited per
+        output point and image with a full chip. A group of more points visits a larger union of
+        slots, a block of more images pads the batch more, fewer rows per workgroup re-read the
+        weights more often but fill the chip where there is little to do. Measured on C2 layers
+        2-4 (B = 256) and on 230 isotropic points with V = 100 (B = 40 and 256): the plan
+        taken is the fastest of eleven or within 8% of it."""
+        img = self._img
+        hit = img.plans.get(batch)
+        if hit is not None:
+            return hit
+        if len(img.plans) >= 64:
+            img.plans.clear()
+        n_out = self.out_coords.shape[0]
+        best = None
+        for rb, cb, eff in ((4, 2, 1.0), (4, 1, 1.25), (2, 2, 1.25), (2, 1, 1.4), (1, 2, 1.7), (1, 1, 2.0)):
+            n_ct = -(-self.out_channels // (128 * cb))
+            eff *= n_ct * 128 * cb / self.out_channels
+            for ib in (16, 32, 64, 128):
+                pp = rb * 32 // ib
+                if pp < 1 or (ib > 16 and ib >= 2 * batch):
+                    continue
+                if pp not in img.unions:
+                    img.unions[pp] = T.image_row_union(img.slot_ptr, self._point_order(), pp)
+                blocks = -(-batch // ib)
+                groups = -(-n_out // pp) * blocks * n_ct
+                fill = -(-groups // 512) * 512 / groups        # two workgroups on each of 256 CUs
+                work = blocks * ib / batch * img.unions[pp] * eff * fill
+                if best is None or work < best[0]:
+                    best = (work, (rb, ib, cb))
+        img.plans[batch] = best
+        return best
+
+    def _point_order(self):
+        """Output points in compact runs, for the image-row kernel's groups: the workgroups that
+        run together then share their input rows in L2 (C3: 3.36 ms with runs of whole rings,
+        2.82 ms with compact ones, and neighbouring points use nearly the same slots)."""
+        if self._img.order is None:
+            c = self.out_coords
+            self._img.order = T.spatial_order(c.cortical if c.cortical is not None else c.cartesian)
+        return self._img.order
+
+    def _image_tables_of(self, pp, device):
+        """The image-row kernel's device tables for groups of ``pp`` points, built once."""
+        hit = self._img.tables.get(pp)
+        if hit is None or hit[0] != device:
+            ent, points, nact = T.image_row_tables(self._img.slot_ptr, self._img.nbr, self.slot_order,
+                                                   self._point_order(), pp)
+            hit = (device, ent.to(device), points.to(device), nact.to(device))
+            self._img.tables[pp] = hit
+        return hit[1:]
+
+    def _packed_weight_image(self, dtype):
+        """``(fragments, non-finite flag, w_scale)`` of the image-row kernel's weight
+        (``fovi_knnconv_pack_weight_img``), cached per weight version."""
+        w = self.weight
+        key = ("image", dtype, w._version, w.data_ptr())
+        hit = self._packed.get(("image", dtype))
+        if hit is not None and hit[0] == key:
+            return hit[1]
+        n_ref = self.ref_coords.shape[0]
+        lib = _lib.load()
+        code = _lib.dtype_code(dtype)
+        src = w.detach().to(torch.float32).contiguous()
+        out = torch.empty(lib.fovi_knnconv_weight_img_elems(self.out_channels, self.in_channels, n_ref, code),
+                          dtype=dtype, device=w.device)
+        flag = torch.zeros(1, dtype=torch.int32, device=w.device)
+        w_scale = self._fp8_weight_scale(src) if dtype == torch.float8_e4m3fn else None
+        _lib.check(lib.fovi_knnconv_pack_weight_img(_lib.ptr(src), self.out_channels, self.in_channels, n_ref,
+                                                    _lib.ptr(out), code, _lib.ptr(self._slot_order_dev),
+                                                    _lib.ptr(w_scale), _lib.ptr(flag), _lib.stream_handle(w.device)),
+                   "fovi_knnconv_pack_weight_img")
+        packed = (out, flag, w_scale)
+        self._packed[("image", dtype)] = (key, packed)
+        return packed
+
+    def _image_path(self, x, dt):
+        """Whether this call runs the image-row kernel: a batch of at least ``IMG_MIN_BATCH`` (below,
+        most of a block of 16 images would be padding), at least 16 input channels, 32-bit
+        offsets within a block of images, and less estimated work than the wide-layer kernel
+        where that one applies. Under stream capture only with its tables already built (their
+        upload cannot be captured)."""
+        bsz = x.shape[0]
+        if not (self.image_rows and bsz >= IMG_MIN_BATCH and self.in_channels >= 16 and self._k <= 32767
+                and x.shape[2] * (-(-self.in_channels // 16) * 16) * min(bsz, 128) * dt.itemsize < 2 ** 31 - 4096):
+            return False
+        work, (rb, ib, _) = self._image_plan(bsz)
+        if dt != torch.float32 and self._mfma_path(x, dt):
+            # the wide-layer kernel visits every slot, one workgroup of 256 points of an image per
+            # CU; a slot costs it 3/4 of the image-row kernel's (C3: 3.2 ms for 25, 2.82 for 16.9)
+            tiles = bsz * -(-self.out_coords.shape[0] // 256) * -(-self.out_channels // 256)
+            pad = -(-self.out_coords.shape[0] // 256) * 256 / self.out_coords.shape[0]
+            if 0.75 * self.ref_coords.shape[0] * pad * (-(-tiles // 256) * 256 / tiles) < work:
+                return False
+        hit = self._img.tables.get(rb * 32 // ib)
+        return (hit is not None and hit[0] == x.device) or not torch.cuda.is_current_stream_capturing()
+
+    def _image_args(self, a, x, dt):
+        """Image-row kernel: the tables and weight into the ``fovi_knnconv_args`` ``a``; returns
+        what its pointers name."""
+        frag, flag, w_scale = self._packed_weight_image(dt)
+        _, (rb, ib, cb) = self._image_plan(x.shape[0])
+        pp = rb * 32 // ib
+        ent, points, nact = self._image_tables_of(pp, x.device)
+        a.w, a.w_dtype, a.w_layout = frag.data_ptr(), _lib.dtype_code(dt), _lib.W_IMG
+        a.k_pad = x.shape[1] * self.ref_coords.shape[0]
+        a.img_ent, a.img_points, a.img_nact = ent.data_ptr(), points.data_ptr(), nact.data_ptr()
+        a.img_flag = flag.data_ptr()
+        a.img_groups, a.img_pp, a.img_ib, a.img_cb = points.shape[0], pp, ib, cb
+        return frag, flag, w_scale, ent, points, nact
+
+    @staticmethod
+    def _image_input(x, dt):
+        """``x`` as channels-last rows of a multiple of 16 bytes, 128 images within 2 GiB (``x``
+        itself where it is)."""
+        al = 16 // dt.itemsize
+        b, c, n = x.shape
+        if (c % al == 0 and x.stride(1) == 1 and x.stride(2) % al == 0 and x.stride(0) % al == 0
+                and x.data_ptr() % 16 == 0
+                and ((min(b, 128) - 1) * x.stride(0) + (n - 1) * x.stride(2) + c) * dt.itemsize < 2 ** 31 - 4096):
+            return x
+        cp = -(-c // al) * al
+        buf = (torch.empty if cp == c else torch.zeros)(b, n, cp, dtype=dt, device=x.device)
+        buf[:, :, :c].copy_(x.transpose(1, 2))
+        return buf.transpose(1, 2)
 
     @property
     def padded_channels(self):
@@ -665,22 +817,29 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
                 buf, view = self.padded_input(x.shape[0], x.device)
                 view.copy_(x)
                 x = view
-        mfma = cp is None and self._mfma_path(x, dt)
-        self.last_weight_layout = "mfma" if mfma else "rows"
-        w = self._packed_weight_mfma() if mfma else self._packed_weight(dt, c_slot)
+        image = cp is None and self._image_path(x, dt)
+        if image:
+            x = self._image_input(x, dt)
+            c_slot = x.shape[1]
+        mfma = cp is None and not image and self._mfma_path(x, dt)
+        self.last_weight_layout = "image" if image else "mfma" if mfma else "rows"
+        w = (None if image else self._packed_weight_mfma() if mfma else self._packed_weight(dt, c_slot))
         bsz, n_out = x.shape[0], self.out_coords.shape[0]
         y = torch.empty(bsz, n_out, self.out_channels, dtype=dt, device=x.device)
         bias = None if self.bias is None else self.bias.detach().to(torch.float32).contiguous()
         a = _lib.KnnConvArgs()
         a.x = x.data_ptr(); a.x_dtype = _lib.dtype_code(dt)
-        a.batch, a.c_in, a.n_in = bsz, self.in_channels, x.shape[2]
+        a.batch, a.c_in, a.n_in = bsz, x.shape[1], x.shape[2]
         a.x_stride[:] = list(x.stride())
         a.n_out, a.k, a.n_ref = n_out, self._k, self.ref_coords.shape[0]
         a.slot_ptr = self.slot_ptr.data_ptr(); a.nbr_sorted = self.nbr_sorted.data_ptr()
-        a.w = w.data_ptr(); a.w_dtype = _lib.dtype_code(dt)
-        a.w_layout = _lib.W_MFMA if mfma else _lib.W_ROWS
+        if image:
+            img = self._image_args(a, x, dt)
+        else:
+            a.w = w.data_ptr(); a.w_dtype = _lib.dtype_code(dt)
+            a.w_layout = _lib.W_MFMA if mfma else _lib.W_ROWS
+            a.k_pad = self.in_channels * self.ref_coords.shape[0] if mfma else w.shape[1]
         a.c_out = self.out_channels
-        a.k_pad = self.in_channels * self.ref_coords.shape[0] if mfma else w.shape[1]
         a.bias = None if bias is None else bias.data_ptr()
         a.y = y.data_ptr(); a.y_dtype = _lib.dtype_code(dt)
         a.y_stride[:] = [y.stride(0), y.stride(2), y.stride(1)]
@@ -688,6 +847,8 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
             raise ValueError(f"activation must be None or 'relu', got {activation!r}")
         a.activation = _lib.ACT_RELU if activation == "relu" else _lib.ACT_NONE
         a.w_c_slot = c_slot
+        if image:
+            return a, y, (x, img, bias)
         vm = None
         if view_major and self.view_major_kernel:
             frag, nb, cb, finite = self._packed_weight_vm(c_slot)
@@ -738,14 +899,16 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         bsz, c, n_in = x.shape
         n_out, v, c_out = self.out_coords.shape[0], self.ref_coords.shape[0], self.out_channels
         dt = x.dtype
-        dy2 = dy.to(dt).permute(0, 2, 1).reshape(bsz * n_out, c_out)
-        w_sm = weight.detach().to(dt).reshape(c_out, c, v).permute(0, 2, 1).reshape(c_out, v * c)
+        dy = dy.to(dt)
+        if dy.stride(1) != 1:       # channels-last once, for every kernel below
+            dy = dy.transpose(1, 2).contiguous().transpose(1, 2)
         lib = _lib.load()
         stream = _lib.stream_handle(x.device)
         dx = dw = None
         if need_w and self.dw_fused and self._dw_fused_ok(x, dt):
             dw = self._dw_fused(x, dy).to(weight.dtype)
         elif need_w:
+            dy2 = dy.permute(0, 2, 1).reshape(bsz * n_out, c_out)
             a_mat = torch.empty(bsz * n_out, v * c, dtype=dt, device=x.device)
             sa = _lib.SlotsumArgs()
             sa.x = x.data_ptr(); sa.x_dtype = _lib.dtype_code(dt); sa.a_dtype = _lib.dtype_code(dt)
@@ -758,8 +921,10 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
             dw_sm = dy2.t() @ a_mat                                     # [C_out, V * C]
             dw = dw_sm.reshape(c_out, v, c).permute(0, 2, 1).reshape(c_out, c * v).to(weight.dtype)
         if need_x and self.dx_by_transposed_conv:
-            dx = self._transposed(x.device)(dy.to(dt), weight)
+            dx = self._transposed(x.device)(dy, weight)
         elif need_x:
+            dy2 = dy.permute(0, 2, 1).reshape(bsz * n_out, c_out)
+            w_sm = weight.detach().to(dt).reshape(c_out, c, v).permute(0, 2, 1).reshape(c_out, v * c)
             g = (dy2 @ w_sm).contiguous()                               # [B * N_out, V * C]
             inv_ptr, inv = self._inverse_tables(x.device)
             dx = (torch.empty(bsz, n_in, c, dtype=dt, device=x.device).transpose(1, 2) if x.stride(1) == 1
@@ -786,7 +951,7 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         ``dw_chunk`` output points and ``dw_images_per_group`` images."""
         bsz, c, n_in = x.shape
         n_out, v, c_out = self.out_coords.shape[0], self.ref_coords.shape[0], self.out_channels
-        dyc = dy.to(torch.bfloat16)
+        dyc = dy
         if not (dyc.stride(1) == 1 and dyc.stride(2) % 8 == 0 and dyc.stride(0) % 8 == 0
                 and dyc.data_ptr() % 16 == 0):
             dyc = dyc.transpose(1, 2).contiguous().transpose(1, 2)
@@ -864,10 +1029,15 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
                              f"got {tuple(x.shape)}")
         if self.tile_lo is None:
             raise NotImplementedError("fp8 kNN-conv needs the tile tables (k <= 255, tile spans <= 65535)")
-        mfma = self._mfma_path(x, torch.float8_e4m3fn)
-        self.last_weight_layout = "mfma" if mfma else "rows"
-        w, w_scale = (self._packed_weight_mfma(torch.float8_e4m3fn) if mfma
-                      else self._packed_weight(torch.float8_e4m3fn))
+        image = (self._image_path(x, torch.float8_e4m3fn) and self.in_channels % 64 == 0
+                 and self._image_input(x, torch.float8_e4m3fn) is x)
+        mfma = not image and self._mfma_path(x, torch.float8_e4m3fn)
+        self.last_weight_layout = "image" if image else "mfma" if mfma else "rows"
+        if image:
+            w = None
+        else:
+            w, w_scale = (self._packed_weight_mfma(torch.float8_e4m3fn) if mfma
+                          else self._packed_weight(torch.float8_e4m3fn))
         bsz, n_out = x.shape[0], self.out_coords.shape[0]
         y = torch.empty(bsz, n_out, self.out_channels, dtype=torch.bfloat16, device=x.device)
         bias = None if self.bias is None else self.bias.detach().to(torch.float32).contiguous()
@@ -878,10 +1048,14 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         a.x_stride[:] = list(x.stride())
         a.n_out, a.k, a.n_ref = n_out, self._k, self.ref_coords.shape[0]
         a.slot_ptr = self.slot_ptr.data_ptr(); a.nbr_sorted = self.nbr_sorted.data_ptr()
-        a.w = w.data_ptr(); a.w_dtype = _lib.F8E4M3
-        a.w_layout = _lib.W_MFMA if mfma else _lib.W_ROWS
+        if image:
+            img = self._image_args(a, x, torch.float8_e4m3fn)
+            w_scale = img[2]
+        else:
+            a.w = w.data_ptr(); a.w_dtype = _lib.F8E4M3
+            a.w_layout = _lib.W_MFMA if mfma else _lib.W_ROWS
+            a.k_pad = self.in_channels * self.ref_coords.shape[0] if mfma else w.shape[1]
         a.c_out = self.out_channels
-        a.k_pad = self.in_channels * self.ref_coords.shape[0] if mfma else w.shape[1]
         a.bias = None if bias is None else bias.data_ptr()
         a.w_scale = w_scale.data_ptr(); a.x_scale_dev = scale.data_ptr()
         a.y = y.data_ptr(); a.y_dtype = _lib.BF16

@@ -1292,3 +1292,65 @@ def stream_slot_order(units_per_slot, rate=256, ahead=3, iters=600, seed=0):
         if c <= best:
             order, best = cand, c
     return order
+
+
+IMG_WINDOW = 256          # consecutive output points the image-row kernel's groups are formed in
+IMG_SAMPLE = 4            # windows looked at when the group size is chosen
+
+
+def spatial_order(coords, leaf=IMG_WINDOW):
+    """A permutation (int32) of the points ``coords [N, D]`` in which every run of about ``leaf``
+    points is compact: recursive median splits along the widest axis."""
+    pts = torch.as_tensor(coords).detach().cpu().to(torch.float64).numpy()
+    out = []
+    stack = [np.arange(pts.shape[0])]
+    while stack:
+        idx = stack.pop()
+        if idx.size <= leaf:
+            out.append(idx)
+            continue
+        sub = pts[idx]
+        axis = int(np.argmax(sub.max(0) - sub.min(0)))
+        half = leaf * (-(-idx.size // leaf) // 2)           # whole leaves on the first side
+        idx = idx[np.argsort(sub[:, axis], kind="stable")]
+        stack += [idx[half:], idx[:half]]
+    return torch.from_numpy(np.concatenate(out)).to(torch.int32)
+
+
+def image_row_tables(slot_ptr, nbr_sorted, order, point_order, pp):
+    """``(ent [G, V, pp, 4], points [G, pp], nact [G])`` (int32, host) of the image-row kernel:
+    groups of ``pp`` output points with similar slot sets and the slots each group visits
+    (``fovi_knnconv_img_tables``). ``order`` is the slot visit order, ``point_order`` the order
+    of the points the groups are formed in; either may be None."""
+    from .. import _lib
+    slot_ptr, nbr_sorted = slot_ptr.cpu().contiguous(), nbr_sorted.cpu().contiguous()
+    n, v = slot_ptr.shape
+    k = nbr_sorted.shape[1]
+    cap = sum(-(-min(IMG_WINDOW, n - w) // pp) for w in range(0, n, IMG_WINDOW))
+    ent = torch.empty(cap, v, pp, 4, dtype=torch.int32)
+    points = torch.empty(cap, pp, dtype=torch.int32)
+    nact = torch.empty(cap, dtype=torch.int32)
+    ordt = None if order is None else torch.tensor(list(order), dtype=torch.int32)
+    got = _lib.load().fovi_knnconv_img_tables(_lib.ptr(slot_ptr), _lib.ptr(nbr_sorted), n, k, v, _lib.ptr(ordt),
+                                              _lib.ptr(point_order), pp, IMG_WINDOW, 1, _lib.ptr(ent),
+                                              _lib.ptr(points), _lib.ptr(nact), None)
+    if got != cap:
+        _lib.check(1, "fovi_knnconv_img_tables")
+    return ent, points, nact
+
+
+def image_row_union(slot_ptr, point_order, pp):
+    """Mean number of slots a group of ``pp`` points visits, from ``IMG_SAMPLE`` windows."""
+    import ctypes
+
+    from .. import _lib
+    slot_ptr = slot_ptr.cpu().contiguous()
+    n, v = slot_ptr.shape
+    windows = -(-n // IMG_WINDOW)
+    mean = ctypes.c_double(0.0)
+    got = _lib.load().fovi_knnconv_img_tables(_lib.ptr(slot_ptr), None, n, 1, v, None, _lib.ptr(point_order), pp,
+                                              IMG_WINDOW, max(1, windows // IMG_SAMPLE), None, None, None,
+                                              ctypes.byref(mean))
+    if got <= 0:
+        _lib.check(1, "fovi_knnconv_img_tables")
+    return mean.value

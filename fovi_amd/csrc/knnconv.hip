@@ -1356,6 +1356,18 @@ extern "C" int fovi_knnconv_fwd(const fovi_knnconv_args* a, void* stream) {
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
 
+  if (a->w_layout == FOVI_W_IMG) {
+    if (!launch_knnconv_img(p, a, s)) {
+      set_error("fovi_knnconv_fwd: the image-row kernel needs channels-last 16-byte input rows of the weight's dtype "
+                "within 2 GiB per image block, its tables and flag, and a %s output",
+                a->x_dtype == FOVI_F32 ? "F32" : "BF16");
+      return 1;
+    }
+    note_path(a->x_dtype == FOVI_F32 ? "f32 image rows" : a->x_dtype == FOVI_BF16 ? "bf16 image rows"
+                                                                                 : "fp8 image rows");
+    return check_launch("fovi_knnconv_fwd(image rows)");
+  }
+
   if (a->w_layout != FOVI_W_ROWS) {
     const int f8 = a->x_dtype == FOVI_F8E4M3 && a->w_dtype == FOVI_F8E4M3;
     if (a->w_layout != FOVI_W_MFMA || !(f8 || (a->x_dtype == FOVI_BF16 && a->w_dtype == FOVI_BF16)) ||

@@ -132,4 +132,7 @@ int v5_tiles_of(const KnnParams& p);
 int launch_knnconv_bf16_v5(const KnnParams& p, int out_t, hipStream_t s);
 int launch_knnconv_fp8_v5(const KnnParams& p, int out_t, hipStream_t s);
 
+// 1 if the image-row kernel (knnconv_img.hip) was launched, 0 if the arguments do not fit it.
+int launch_knnconv_img(const KnnParams& p, const fovi_knnconv_args* a, hipStream_t s);
+
 }  // namespace fovi

@@ -23,13 +23,13 @@
 extern "C" {
 #endif
 
-#define FOVI_ABI_VERSION 33
+#define FOVI_ABI_VERSION 34
 
 enum fovi_dtype { FOVI_F32 = 0, FOVI_BF16 = 1, FOVI_F8E4M3 = 2 };
 enum fovi_interp { FOVI_NEAREST = 0, FOVI_BILINEAR = 1 };
 enum fovi_padding { FOVI_PAD_ZEROS = 0, FOVI_PAD_BORDER = 1 };
 enum fovi_activation { FOVI_ACT_NONE = 0, FOVI_ACT_RELU = 1 };
-enum fovi_weight_layout { FOVI_W_ROWS = 0, FOVI_W_MFMA = 1 };
+enum fovi_weight_layout { FOVI_W_ROWS = 0, FOVI_W_MFMA = 1, FOVI_W_IMG = 2 };
 
 /* Version of this header the library was built from (FOVI_ABI_VERSION). */
 int fovi_abi_version(void);
@@ -269,6 +269,24 @@ typedef struct fovi_knnconv_args {
   const void* vm_w;
   int32_t vm_nb;
   int32_t vm_cb;
+  /*
+   * The image-row kernel (w_layout = FOVI_W_IMG, weight from fovi_knnconv_pack_weight_img): F32,
+   * BF16 or F8E4M3 input of the weight's dtype, channels-last rows of a multiple of 16 bytes,
+   * 16-byte aligned; y F32 (F32 input) or BF16. A workgroup takes img_pp points x img_ib images
+   * (img_ib a power of two in 16 .. 128, img_pp * img_ib = 32, 64 or 128) and visits only the
+   * slots its points use; tables from fovi_knnconv_img_tables with pp = img_pp:
+   *   img_ent [img_groups, n_ref, img_pp] 16-byte entries, img_points [img_groups, img_pp],
+   *   img_nact [img_groups]; img_flag: the flag the weight packing wrote; img_cb: 32-column
+   *   blocks per wave (1 or 2).
+   */
+  const uint32_t* img_ent;
+  const int32_t* img_points;
+  const int32_t* img_nact;
+  const int32_t* img_flag;
+  int64_t img_groups;
+  int32_t img_pp, img_ib;
+  int32_t img_cb;
+  int32_t reserved8;
 } fovi_knnconv_args;
 
 int fovi_knnconv_fwd(const fovi_knnconv_args* args, void* stream);
@@ -359,6 +377,35 @@ int64_t fovi_knnconv_weight_mfma_elems(int64_t c_out, int64_t c_in, int64_t n_re
 int fovi_knnconv_pack_weight_mfma(const float* w_ref, int64_t c_out, int64_t c_in, int64_t n_ref,
                                   void* w_frag, int32_t out_dtype, const int32_t* slot_order,
                                   const float* w_scale, void* stream);
+
+/*
+ * Weight of the image-row kernel (w_layout = FOVI_W_IMG) for dtype F32, BF16 or F8E4M3 (divided
+ * by w_scale[o], RNE, saturating): fovi_knnconv_weight_img_elems() elements in 1 KB fragments
+ * f = (it * ncb + cb) * 2 + h, ncb = 2 * ceil(c_out / 64), it = chunk * n_ref + p, chunks of 16,
+ * 32 or 64 channels, position p of the slot visit order (slot_order, device, or NULL: 0, 1, ...).
+ * Lane l of fragment f holds w_ref[o = 32 * cb + l % 32][c * n_ref + v] (zero for o >= c_out or
+ * c >= c_in), channel of the chunk 8 h + 4 (l / 32) + e (F32), 16 h + 8 (l / 32) + e (BF16),
+ * 32 (l / 32) + 16 h + e (F8E4M3). *flag (device, zeroed by the caller) is set when a packed value
+ * is not finite.
+ */
+int64_t fovi_knnconv_weight_img_elems(int64_t c_out, int64_t c_in, int64_t n_ref, int32_t dtype);
+int fovi_knnconv_pack_weight_img(const float* w_ref, int64_t c_out, int64_t c_in, int64_t n_ref, void* w_frag,
+                                 int32_t dtype, const int32_t* slot_order, const float* w_scale, int32_t* flag,
+                                 void* stream);
+
+/*
+ * Host tables of the image-row kernel (all pointers host memory): groups of pp output points
+ * with similar slot sets, formed within windows of `window` consecutive points of point_order (a
+ * permutation of the points, or NULL: the index order). Writes, per
+ * group, its points (-1: none), the number of slots its points use, and n_ref * pp entries of 4 words
+ * {neighbour 1, neighbour 2 (0x80000000: none), count << 16 | begin, position} with the used slots first, each part in visit order. Returns the number of groups (at most
+ * (n_out / window + 1) * ceil(window / pp)), -1 on bad arguments. With ent NULL nothing is
+ * written and only every stride-th window is grouped; *mean_union (optional) gets the mean number
+ * of used slots per group.
+ */
+int64_t fovi_knnconv_img_tables(const int32_t* slot_ptr, const int32_t* nbr, int64_t n_out, int64_t k, int64_t n_ref,
+                                const int32_t* slot_order, const int32_t* point_order, int32_t pp, int64_t window,
+                                int64_t stride, uint32_t* ent, int32_t* points, int32_t* nact, double* mean_union);
 
 /*
  * Per-tensor OCP e4m3 quantization of activations for the fp8 kNN-conv path
