@@ -393,7 +393,7 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         self.dw_fused = True
         # its work split: output points per pair segment, images per workgroup
         self.dw_chunk = 1 << 30
-        self.dw_images_per_group = 1
+        self.dw_images_per_group = None      # None: _dw_split
         # wide layers (bf16 c_in % 32 == 0 or e4m3 c_in % 64 == 0, c_out filling >= 3/4 of its
         # 256-channel tiles, tables within LDS): weights in MFMA-fragment order for the
         # 256 x 256-tile kernel (False: the row-packed kernels)
@@ -948,7 +948,7 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
     def _dw_fused(self, x, dy):
         """``dW`` (fp32, reference layout) by ``fovi_knnconv_dw``: per slot a GEMM over its
         (output, input) pairs, no slot-sum matrix; one workgroup per slot, chunk of
-        ``dw_chunk`` output points and ``dw_images_per_group`` images."""
+        ``dw_chunk`` output points and ``dw_images_per_group`` images (None: ``_dw_split``)."""
         bsz, c, n_in = x.shape
         n_out, v, c_out = self.out_coords.shape[0], self.ref_coords.shape[0], self.out_channels
         dyc = dy
@@ -958,7 +958,7 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         pair_off, pairs = self._slot_pairs(x.device)
         lib = _lib.load()
         n_chunks = (pair_off.numel() - 1) // v
-        ipg = self.dw_images_per_group
+        ipg = self.dw_images_per_group or self._dw_split(bsz, pair_off.numel() - 1)
         nbytes = lib.fovi_knnconv_dw_workspace_bytes(bsz, ipg, n_chunks, c, c_out, v)
         ws = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
         dw = torch.empty(c_out, c * v, dtype=torch.float32, device=x.device)
@@ -973,6 +973,33 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         a.dw = dw.data_ptr()
         _lib.check(lib.fovi_knnconv_dw(a, _lib.stream_handle(x.device)), "fovi_knnconv_dw")
         return dw
+
+    def _dw_split(self, batch, segments):
+        """Images per workgroup of ``fovi_knnconv_dw``: the split with the least estimated time. More
+        groups fill the chip more evenly (one workgroup per CU with 256 x 256 channel tiles,
+        two or more with smaller ones), but each writes a partial tile of every slot, which is
+        read again: one group per image cost 96 -> 256 channels with V = 100 at 256 images
+        1.68 ms (2.5 GB of partials of one 57-pair step each). Below, a step's time is
+        that of 64 pairs on a 256 x 256 tile (4.1 us on the 256 -> 256 layer, C3), the last
+        round is a whole one (slots differ in length), a partial tile's time is two passes over
+        it at 4 TB/s. Measured: V = 100, 256 images 1305, 505, 316, 440, 740 us for 1, 4, 16, 64,
+        128 images; V = 25, 64 images 119, 115, 119, 184 for 1, 2, 4, 8; C3 1.9 and 2.2 ms for 1
+        and 2 of 16 images."""
+        tile = [128 if c <= 128 else 256 for c in (self.out_channels, self.in_channels)]
+        tiles = -(-self.out_channels // tile[0]) * -(-self.in_channels // tile[1])
+        area = tile[0] * tile[1] / 65536
+        slots = 256 * max(1, int(1 / area))
+        steps = self.nbr_sorted.numel() / 64 / segments        # 64-pair steps per segment and image
+        best = None
+        groups = 1
+        while groups <= batch:
+            ipg = -(-batch // groups)
+            n = -(-batch // ipg) * segments * tiles
+            t = (n / slots + 1) * ipg * max(1.0, steps) * 4.1 + n * area * 65536 * 8 / 4e6
+            if best is None or t < best[0]:
+                best = (t, ipg)
+            groups = max(groups + 1, groups * 9 // 8)
+        return best[1]
 
     def _slot_pairs(self, device):
         """``knn_tables.slot_pairs`` of this layer, built on the first backward and kept."""

@@ -4,17 +4,19 @@
 // neighbour i sits in slot v of n of dy[b, n, o] * x[b, i, c]: for every slot a GEMM whose
 // reduction runs over that slot's pair list (the sum of a collision slot is linear, so its
 // pairs enter one by one). The pairs come in segments (one slot, one chunk of output
-// points); a workgroup owns one segment, a group of images and one 256 x 256 (o, c) tile.
-// Its eight waves, two per SIMD so one wave's memory waits overlap the other's MFMAs, hold
-// 128 x 64 fp32 blocks (8 blocks of v_mfma_f32_32x32x16_bf16). Workgroups are numbered
-// slot-fastest and mapped XCD by XCD, so the V workgroups of a chunk share one L2.
+// points); a workgroup owns one segment, a group of images and one TO x TC (o, c) tile: 256
+// channels, or 128 where the layer has no more (96 x 256 channels on a 256 x 256 tile spend
+// 62% of the products on zeros). Its waves hold 128 x 64 fp32 blocks (8 blocks of
+// v_mfma_f32_32x32x16_bf16): eight of them, two per SIMD so one wave's memory waits overlap
+// the other's MFMAs, or two workgroups of four (or four of two) per CU. Workgroups are
+// numbered slot-fastest and mapped XCD by XCD, so the V workgroups of a chunk share one L2.
 //
-// Per step of 64 pairs the workgroup loads the 64 dy rows and the 64 x rows (16-byte
-// chunks, a full row per 32 lanes) into LDS in their natural [pair][channel] layout, double
-// buffered one step ahead. Both MFMA operands need the pair index contiguous per lane, which
+// Per step of K = 64 pairs (32 with the smaller tiles) the workgroup loads the dy rows and the x
+// rows (16-byte chunks, a full row per 32 or 16 lanes) into LDS in their natural
+// [pair][channel] layout, double buffered one step ahead. Both MFMA operands need the pair index contiguous per lane, which
 // the transposed LDS read ds_read_b64_tr_b16 delivers: within a 16-lane group, lane j
 // addresses four channels of pair row k0 + j/4 and lane i receives channel i of pairs
-// k0 .. k0 + 3. Rows are 576 bytes apart so those reads hit 64 distinct banks.
+// k0 .. k0 + 3. Rows are 576 (320) bytes apart so those reads hit 64 distinct banks.
 // Per-workgroup partial tiles go to a caller workspace; a second kernel sums them into the
 // reference weight layout (column c * V + v), fp32.
 #include "common.h"
@@ -22,12 +24,18 @@
 namespace fovi {
 namespace {
 
-constexpr int DW_T = 256;          // o and c tile
-constexpr int DW_K = 64;           // pairs per step
-constexpr int DW_R = DW_K / 16;    // rows per thread and operand in a step (512 threads, 32 per row)
-constexpr int DW_RS = 576;         // LDS bytes per pair row (256 bf16 + 64 bytes of bank skew)
-constexpr int DW_BUF = DW_K * DW_RS;            // one operand, one step
-constexpr int DW_LDS = 2 * 2 * DW_BUF;          // two operands, two steps: 147,456 bytes
+// Tile of the output (O) or input (C) channels: 256, or 128 for up to 128 channels.
+inline int64_t dw_tile(int64_t channels) { return channels <= 128 ? 128 : 256; }
+
+template <int TO, int TC> struct DwTile {
+  static constexpr int NT = (TO / 128) * (TC / 64) * 64;       // threads: a wave per 128 x 64 block
+  static constexpr int K = TO == 256 && TC == 256 ? 64 : 32;   // pairs per step
+  static constexpr int GO = TO / 8, GC = TC / 8;               // 16-byte chunks per row
+  static constexpr int RO = K * GO / NT, RC = K * GC / NT;     // rows per thread and step
+  static constexpr int SO = TO * 2 + 64, SC = TC * 2 + 64;     // LDS bytes per row (64 bytes of bank skew)
+  static constexpr int BUF = K * (SO + SC);                    // one step
+  static constexpr int LDS = 2 * BUF;                          // 256 x 256: 147,456 bytes
+};
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
@@ -41,8 +49,8 @@ struct DwParams {
   int64_t B, C, Cout, Nin, Nout, V;
   const int32_t* pair_off;         // [NQ * V + 1], segment q * V + v
   const int32_t* pairs;            // (n, i) per pair; n < 0 pads
-  int64_t NQ, ipg, S, tiles_o, tiles_c;
-  float* part;                     // [S, NQ, V, tiles_o, tiles_c, 256, 256]
+  int64_t NQ, ipg, S, tiles_o, tiles_c, to, tc;
+  float* part;                     // [S, NQ, V, tiles_o, tiles_c, to, tc]
 };
 
 __device__ __forceinline__ s16x4 tr_read(const uint8_t* lds_base, int byte_off) {
@@ -50,7 +58,10 @@ __device__ __forceinline__ s16x4 tr_read(const uint8_t* lds_base, int byte_off) 
       (__attribute__((address_space(3))) s16x4*)(reinterpret_cast<uintptr_t>(lds_base) + byte_off));
 }
 
-__global__ __launch_bounds__(512, 1) void knnconv_dw_kernel(DwParams p, int64_t total, int64_t padded) {
+template <int TO, int TC>
+__global__ __launch_bounds__((DwTile<TO, TC>::NT), (TO == 256 && TC == 256 ? 1 : 2)) void knnconv_dw_kernel(
+    DwParams p, int64_t total, int64_t padded) {
+  typedef DwTile<TO, TC> D;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int64_t L = xcd_tile(blockIdx.x, padded);
   if (L >= total) return;                       // whole workgroup: before any barrier
@@ -62,21 +73,22 @@ __global__ __launch_bounds__(512, 1) void knnconv_dw_kernel(DwParams p, int64_t 
   rest /= p.tiles_o;
   const int64_t q = rest % p.NQ;
   const int64_t split = rest / p.NQ;
-  const int64_t o0 = to * DW_T, c0 = tc * DW_T;
+  const int64_t o0 = to * TO, c0 = tc * TC;
 
-  // eight waves, two per SIMD: wave (wm, wn) holds o rows wm*128 .. +127, c columns wn*64 .. +63
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wm = wave >> 2, wn = wave & 3;
+  // wave (wm, wn) holds o rows wm*128 .. +127, c columns wn*64 .. +63
+  constexpr int WN = TC / 64;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wm = wave / WN, wn = wave % WN;
   const int64_t seg = q * p.V + v;
   const int64_t P0 = p.pair_off[seg], P1 = p.pair_off[seg + 1];
-  const int64_t steps_img = (P1 - P0 + DW_K - 1) / DW_K;     // the last step's tail reads as pads
+  const int64_t steps_img = (P1 - P0 + D::K - 1) / D::K;     // the last step's tail reads as pads
   const int64_t b_beg = split * p.ipg;
   const int64_t steps = steps_img * (min(p.B, b_beg + p.ipg) - b_beg);
 
-  // load task: pair rows t/32 + 16r (r < DW_R), 16-byte chunk g of the row; chunks past the
-  // channels load chunk 0 and pads load row 0, both masked to zero when stored
-  const int g = t & 31, pr0 = t >> 5;
-  const bool okc = c0 + 8 * g < p.C, oko = o0 + 8 * g < p.Cout;
-  const int gd = oko ? g : 0, gc = okc ? g : 0;
+  // load task: dy rows t/GO + (NT/GO) r, 16-byte chunk t%GO of the row, x rows alike; chunks past
+  // the channels load chunk 0 and pads load row 0, both masked to zero when stored
+  const int go = t % D::GO, po = t / D::GO, gc = t % D::GC, pc = t / D::GC;
+  const bool oko = o0 + 8 * go < p.Cout, okc = c0 + 8 * gc < p.C;
+  const int go1 = oko ? go : 0, gc1 = okc ? gc : 0;
 
   f32x16 acc[4][2];
 #pragma unroll
@@ -86,17 +98,21 @@ __global__ __launch_bounds__(512, 1) void knnconv_dw_kernel(DwParams p, int64_t 
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  int2 pe[DW_R];                                // pair entries of the step being prefetched
-  u32x4v rd[DW_R], rx[DW_R];                    // rows of the step in flight
+  int2 eo[D::RO], ec[D::RC];                    // pair entries of the step being prefetched (square tiles: eo)
+  u32x4v rd[D::RO], rx[D::RC];                  // rows of the step in flight
   uint32_t m = 0;                               // their live bits
   auto load_pairs = [&](int64_t st) __attribute__((always_inline)) {
-    const int64_t base = P0 + DW_K * ((st < steps ? st : 0) % steps_img);
+    const int64_t base = P0 + D::K * ((st < steps ? st : 0) % steps_img);
+    auto entry = [&](int64_t pi) {
+      int2 e = *reinterpret_cast<const int2*>(p.pairs + 2 * (pi < P1 ? pi : P1 - 1));
+      if (pi >= P1) e.x = -1;                     // past the segment: a pad
+      return e;
+    };
 #pragma unroll
-    for (int r = 0; r < DW_R; ++r) {
-      const int64_t pi = base + pr0 + 16 * r;
-      pe[r] = *reinterpret_cast<const int2*>(p.pairs + 2 * (pi < P1 ? pi : P1 - 1));
-      if (pi >= P1) pe[r].x = -1;                 // past the segment: a pad
-    }
+    for (int r = 0; r < D::RO; ++r) eo[r] = entry(base + po + (D::NT / D::GO) * r);
+    if constexpr (D::GO != D::GC)
+#pragma unroll
+      for (int r = 0; r < D::RC; ++r) ec[r] = entry(base + pc + (D::NT / D::GC) * r);
   };
   auto load_rows = [&](int64_t st) __attribute__((always_inline)) {
     const bool on = st < steps;
@@ -104,31 +120,40 @@ __global__ __launch_bounds__(512, 1) void knnconv_dw_kernel(DwParams p, int64_t 
     const uint16_t* xb = p.x + b * p.xs0 + c0;
     const uint16_t* db = p.dy + b * p.ds0 + o0;
     m = 0;
+    // 32-bit element offsets within the image (the host checks they fit)
 #pragma unroll
-    for (int r = 0; r < DW_R; ++r) {
-      const bool live = on && pe[r].x >= 0;
-      const uint32_t n = live ? pe[r].x : 0, i = live ? pe[r].y : 0;
-      // 32-bit element offsets within the image (the host checks they fit)
-      rd[r] = *reinterpret_cast<const u32x4v*>(db + (n * static_cast<uint32_t>(p.ds2) + 8u * gd));
-      rx[r] = *reinterpret_cast<const u32x4v*>(xb + (i * static_cast<uint32_t>(p.xs2) + 8u * gc));
-      m |= static_cast<uint32_t>(live && oko) << r | static_cast<uint32_t>(live && okc) << (DW_R + r);
+    for (int r = 0; r < D::RO; ++r) {
+      const bool live = on && eo[r].x >= 0;
+      const uint32_t n = live ? eo[r].x : 0;
+      rd[r] = *reinterpret_cast<const u32x4v*>(db + (n * static_cast<uint32_t>(p.ds2) + 8u * go1));
+      m |= static_cast<uint32_t>(live && oko) << r;
+    }
+#pragma unroll
+    for (int r = 0; r < D::RC; ++r) {
+      const int2 e = D::GO == D::GC ? eo[r] : ec[r];
+      const bool live = on && e.x >= 0;
+      const uint32_t i = live ? e.y : 0;
+      rx[r] = *reinterpret_cast<const u32x4v*>(xb + (i * static_cast<uint32_t>(p.xs2) + 8u * gc1));
+      m |= static_cast<uint32_t>(live && okc) << (D::RO + r);
     }
   };
   auto store_rows = [&](int buf) __attribute__((always_inline)) {
-    uint8_t* bd = smem + buf * 2 * DW_BUF;
-    uint8_t* bx = bd + DW_BUF;
+    uint8_t* bd = smem + buf * D::BUF;
+    uint8_t* bx = bd + D::K * D::SO;
     const u32x4v z = {0, 0, 0, 0};
 #pragma unroll
-    for (int r = 0; r < DW_R; ++r) {
-      *reinterpret_cast<u32x4v*>(bd + (pr0 + 16 * r) * DW_RS + 16 * g) = (m >> r & 1) ? rd[r] : z;
-      *reinterpret_cast<u32x4v*>(bx + (pr0 + 16 * r) * DW_RS + 16 * g) = (m >> (DW_R + r) & 1) ? rx[r] : z;
-    }
+    for (int r = 0; r < D::RO; ++r)
+      *reinterpret_cast<u32x4v*>(bd + (po + (D::NT / D::GO) * r) * D::SO + 16 * go) = (m >> r & 1) ? rd[r] : z;
+#pragma unroll
+    for (int r = 0; r < D::RC; ++r)
+      *reinterpret_cast<u32x4v*>(bx + (pc + (D::NT / D::GC) * r) * D::SC + 16 * gc) = (m >> (D::RO + r) & 1) ? rx[r] : z;
   };
 
   // this lane's transposed-read offsets: 16-lane group G supplies pair rows kb*16 + 8*(G>>1)
   // + li/4 (+4 for the second half) and channels 16*(G&1) + 4*(li%4) of each 32-block
   const int G = lane >> 4, li = lane & 15;
-  const int lane_off = ((G >> 1) * 8 + (li >> 2)) * DW_RS + ((G & 1) * 16 + 4 * (li & 3)) * 2;
+  const int lrow = (G >> 1) * 8 + (li >> 2), lcol = ((G & 1) * 16 + 4 * (li & 3)) * 2;
+  const int off_d = lrow * D::SO + lcol + wm * 256, off_x = lrow * D::SC + lcol + wn * 128;
 
   if (steps > 0) {
     // prologue: step 0 into LDS buffer 0, step 1 in flight, pair entries of step 2 loading
@@ -140,21 +165,21 @@ __global__ __launch_bounds__(512, 1) void knnconv_dw_kernel(DwParams p, int64_t 
     load_pairs(2);
     __syncthreads();
     for (int64_t st = 0; st < steps; ++st) {
-      const uint8_t* bd = smem + (st & 1) * 2 * DW_BUF;
-      const uint8_t* bx = bd + DW_BUF;
+      const uint8_t* bd = smem + (st & 1) * D::BUF;
+      const uint8_t* bx = bd + D::K * D::SO;
 #pragma unroll
-      for (int kb = 0; kb < DW_K / 16; ++kb) {
+      for (int kb = 0; kb < D::K / 16; ++kb) {
         bf16x8 af[4], bf[2];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int off = lane_off + kb * 16 * DW_RS + (wm * 128 + i * 32) * 2;
-          const s16x4 lo = tr_read(bd, off), hi = tr_read(bd, off + 4 * DW_RS);
+          const int off = off_d + kb * 16 * D::SO + i * 64;
+          const s16x4 lo = tr_read(bd, off), hi = tr_read(bd, off + 4 * D::SO);
           af[i] = __builtin_bit_cast(bf16x8, s16x8(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)));
         }
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          const int off = lane_off + kb * 16 * DW_RS + (wn * 64 + j * 32) * 2;
-          const s16x4 lo = tr_read(bx, off), hi = tr_read(bx, off + 4 * DW_RS);
+          const int off = off_x + kb * 16 * D::SC + j * 64;
+          const s16x4 lo = tr_read(bx, off), hi = tr_read(bx, off + 4 * D::SC);
           bf[j] = __builtin_bit_cast(bf16x8, s16x8(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)));
         }
 #pragma unroll
@@ -170,7 +195,7 @@ __global__ __launch_bounds__(512, 1) void knnconv_dw_kernel(DwParams p, int64_t 
     }
   }
 
-  float* out = p.part + (((split * p.NQ * p.V + seg) * p.tiles_o + to) * p.tiles_c + tc) * (DW_T * DW_T);
+  float* out = p.part + (((split * p.NQ * p.V + seg) * p.tiles_o + to) * p.tiles_c + tc) * (TO * TC);
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -179,37 +204,59 @@ __global__ __launch_bounds__(512, 1) void knnconv_dw_kernel(DwParams p, int64_t 
       for (int r = 0; r < 16; ++r) {
         const int o = wm * 128 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
         const int c = wn * 64 + j * 32 + (lane & 31);
-        out[o * DW_T + c] = acc[i][j][r];
+        if (o0 + o < p.Cout && c0 + c < p.C) out[o * TC + c] = acc[i][j][r];   // the reduction reads no others
       }
 }
 
-// dW[o, c * V + v] = sum over the (image group, chunk) partial tiles (fp32); one thread per
-// (v, o, c), consecutive threads along c (coalesced partial reads)
-__global__ __launch_bounds__(256) void knnconv_dw_reduce_kernel(DwParams p, float* dw) {
-  const int64_t total = p.V * p.Cout * p.C;
-  for (int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; q < total;
-       q += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const int64_t c = q % p.C;
-    const int64_t o = (q / p.C) % p.Cout;
-    const int64_t v = q / (p.C * p.Cout);
-    const int64_t tile = (o / DW_T) * p.tiles_c + c / DW_T;
-    const int64_t in_tile = (o % DW_T) * DW_T + c % DW_T;
-    const int64_t stride = p.V * p.tiles_o * p.tiles_c * (DW_T * DW_T);   // next (group, chunk)
-    const float* src = p.part + (v * p.tiles_o * p.tiles_c + tile) * (DW_T * DW_T) + in_tile;
-    // partials added in (group, chunk) order; four loads in flight per trip
-    float sum = 0.0f;
-    const int64_t n = p.S * p.NQ;
-    int64_t sq = 0;
-    for (; sq + 4 <= n; sq += 4) {
-      float t[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) t[u] = src[(sq + u) * stride];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) sum += t[u];
-    }
-    for (; sq < n; ++sq) sum += src[sq * stride];
-    dw[o * p.C * p.V + c * p.V + v] = sum;
+template <int TO, int TC>
+int launch_dw(const DwParams& p, int64_t total, int64_t padded, hipStream_t s) {
+  if (reserve_dynamic_lds(reinterpret_cast<const void*>(&knnconv_dw_kernel<TO, TC>), DwTile<TO, TC>::LDS) != hipSuccess) {
+    set_error("fovi_knnconv_dw: cannot reserve %d bytes of LDS", DwTile<TO, TC>::LDS);
+    return 1;
   }
+  hipLaunchKernelGGL((knnconv_dw_kernel<TO, TC>), dim3(static_cast<unsigned>(padded)), dim3(DwTile<TO, TC>::NT),
+                     (DwTile<TO, TC>::LDS), s, p, total, padded);
+  return check_launch("fovi_knnconv_dw");
+}
+
+// dW[o, c * V + v] = sum over the (image group, chunk) partial tiles (fp32, in that order; four
+// loads in flight per trip). A block takes one o and cc channels: a thread reads along c (the
+// partials' fast axis), the sums go through LDS and leave as runs of cc * V consecutive floats
+// (written straight from the reading order, one float per 4 V bytes, every line of dW is
+// touched V times).
+__global__ __launch_bounds__(256) void knnconv_dw_reduce_kernel(DwParams p, float* dw, int cc, int ccs) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  float* out = reinterpret_cast<float*>(smem);                 // [cc][V]
+  const int V = static_cast<int>(p.V);
+  const int64_t nc = (p.C + cc - 1) / cc;
+  const int64_t o = blockIdx.x / nc, c0 = (blockIdx.x % nc) * cc;
+  const int lc = threadIdx.x & (cc - 1), v0 = threadIdx.x >> ccs, dv = 256 >> ccs;
+  const int64_t c = c0 + lc;
+  const int64_t n = p.S * p.NQ;
+  const int64_t stride = p.V * p.tiles_o * p.tiles_c * (p.to * p.tc);   // next (group, chunk)
+  if (c < p.C) {
+    const int64_t tile = (o / p.to) * p.tiles_c + c / p.tc;
+    const float* base = p.part + tile * (p.to * p.tc) + (o % p.to) * p.tc + c % p.tc;
+    for (int v = v0; v < V; v += dv) {
+      const float* src = base + v * p.tiles_o * p.tiles_c * (p.to * p.tc);
+      float sum = 0.0f;
+      int64_t sq = 0;
+      for (; sq + 4 <= n; sq += 4) {
+        float t[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) t[u] = src[(sq + u) * stride];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) sum += t[u];
+      }
+      for (; sq < n; ++sq) sum += src[sq * stride];
+      out[lc * V + v] = sum;
+    }
+  }
+  __syncthreads();
+  const int64_t left = p.C - c0;
+  const int count = static_cast<int>(left < cc ? left : cc) * V;
+  float* dst = dw + (o * p.C + c0) * p.V;
+  for (int i = threadIdx.x; i < count; i += 256) dst[i] = out[i];
 }
 
 }  // namespace
@@ -221,8 +268,9 @@ extern "C" int64_t fovi_knnconv_dw_workspace_bytes(int64_t batch, int64_t images
                                                    int64_t c_in, int64_t c_out, int64_t n_ref) {
   if (batch < 1 || images_per_group < 1 || n_chunks < 1 || c_in < 1 || c_out < 1 || n_ref < 1) return -1;
   const int64_t splits = (batch + images_per_group - 1) / images_per_group;
-  const int64_t tiles = ((c_out + DW_T - 1) / DW_T) * ((c_in + DW_T - 1) / DW_T);
-  return splits * n_chunks * n_ref * tiles * DW_T * DW_T * static_cast<int64_t>(sizeof(float));
+  const int64_t to = dw_tile(c_out), tc = dw_tile(c_in);
+  const int64_t tiles = ((c_out + to - 1) / to) * ((c_in + tc - 1) / tc);
+  return splits * n_chunks * n_ref * tiles * to * tc * static_cast<int64_t>(sizeof(float));
 }
 
 extern "C" int fovi_knnconv_dw(const fovi_knnconv_dw_args* a, void* stream) {
@@ -259,20 +307,29 @@ extern "C" int fovi_knnconv_dw(const fovi_knnconv_dw_args* a, void* stream) {
   p.B = a->batch; p.C = a->c_in; p.Cout = a->c_out; p.Nin = a->n_in; p.Nout = a->n_out; p.V = a->n_ref;
   p.pair_off = a->pair_off; p.pairs = a->pairs;
   p.NQ = a->n_chunks; p.ipg = a->images_per_group; p.S = (p.B + p.ipg - 1) / p.ipg;
-  p.tiles_o = (p.Cout + DW_T - 1) / DW_T; p.tiles_c = (p.C + DW_T - 1) / DW_T;
+  p.to = dw_tile(p.Cout); p.tc = dw_tile(p.C);
+  p.tiles_o = (p.Cout + p.to - 1) / p.to; p.tiles_c = (p.C + p.tc - 1) / p.tc;
   p.part = static_cast<float*>(a->workspace);
   const int64_t total = p.S * p.NQ * p.V * p.tiles_o * p.tiles_c;
   const int64_t padded = (total + 7) / 8 * 8;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (reserve_dynamic_lds(reinterpret_cast<const void*>(&knnconv_dw_kernel), DW_LDS) != hipSuccess) {
-    set_error("fovi_knnconv_dw: cannot reserve %d bytes of LDS", DW_LDS);
+  const int rc = p.to == 256 ? (p.tc == 256 ? launch_dw<256, 256>(p, total, padded, s) : launch_dw<256, 128>(p, total, padded, s))
+                             : (p.tc == 256 ? launch_dw<128, 256>(p, total, padded, s) : launch_dw<128, 128>(p, total, padded, s));
+  if (rc) return rc;
+  // channels per reduction block: 32, fewer where their V sums pass 64 KB of LDS
+  int ccs = 5;
+  while (ccs > 0 && (p.V << ccs) * 4 > 64 * 1024) --ccs;
+  const int64_t lds = (p.V << ccs) * 4, blocks = p.Cout * ((p.C + (1 << ccs) - 1) >> ccs);
+  if (lds > 160 * 1024 || blocks > 0x7fffffff) {
+    set_error("fovi_knnconv_dw: n_ref=%lld too large", (long long)p.V);
     return 1;
   }
-  hipLaunchKernelGGL(knnconv_dw_kernel, dim3(static_cast<unsigned>(padded)), dim3(512), DW_LDS, s, p, total,
-                     padded);
-  if (check_launch("fovi_knnconv_dw")) return 1;
-  const int64_t n = p.V * p.Cout * p.C;
-  hipLaunchKernelGGL(knnconv_dw_reduce_kernel, dim3(static_cast<unsigned>(std::min<int64_t>((n + 255) / 256, 65536))),
-                     dim3(256), 0, s, p, a->dw);
+  if (lds > 64 * 1024 &&
+      reserve_dynamic_lds(reinterpret_cast<const void*>(&knnconv_dw_reduce_kernel), static_cast<size_t>(lds)) != hipSuccess) {
+    set_error("fovi_knnconv_dw: cannot reserve %lld bytes of LDS", (long long)lds);
+    return 1;
+  }
+  hipLaunchKernelGGL(knnconv_dw_reduce_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), static_cast<size_t>(lds),
+                     s, p, a->dw, 1 << ccs, ccs);
   return check_launch("fovi_knnconv_dw(reduce)");
 }
