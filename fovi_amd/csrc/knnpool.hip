@@ -11,6 +11,9 @@
 //    loads and store 16-byte output pieces; consecutive points share
 //    neighbours, and each XCD takes a contiguous range of batch rows, so
 //    the rows are fetched into one L2.
+//  * Channel planes (unit point stride: what batch norm returns): one thread per (batch row, output
+//    point, 8 channels), lanes along the points: the thread's neighbour indices are read once
+//    for its 8 planes, the gathers of a wave stay inside one plane row, stores are runs of points.
 //  * Any other strides: one thread per (batch row, output point, channel).
 #include "common.h"
 
@@ -249,6 +252,76 @@ __global__ __launch_bounds__(256) void knnpool_rows_kf_kernel(PoolParams p, uint
   }
 }
 
+// Channel planes, lists of at most POOL_KF neighbours: thread = (batch row, PL_U consecutive
+// channels, output point), a block 2^ls points x 256 / 2^ls channel groups. Bound by the scattered 2- and 4-byte
+// loads, one per neighbour and output, from rows of a few hundred bytes that stay in L1. The
+// reduction is that of the rows kernel. 256 images x 256 channels, 230 -> 60 points, k = 9, bf16:
+// 49 us; 167 us with a thread per output and lanes along the channels (each lane another plane). Its
+// backward, state and dx: 63 + 46 us; 139 + 218 us that way.
+constexpr int PL_U = 8;
+
+template <typename InT, typename OutT, int MODE>
+__global__ __launch_bounds__(256) void knnpool_planes_kernel(PoolParams p, int ls, uint32_t n_tiles, uint32_t groups,
+                                                             uint32_t total_groups) {
+  const uint32_t lane = threadIdx.x & ((1u << ls) - 1);
+  const uint32_t n = ((blockIdx.x % n_tiles) << ls) + lane;
+  const uint32_t cg = (blockIdx.x / n_tiles) * (256u >> ls) + (threadIdx.x >> ls);
+  if (n >= static_cast<uint32_t>(p.Nout) || cg >= total_groups) return;
+  const uint32_t b = cg / groups, c0 = (cg % groups) * PL_U;
+  const int K = static_cast<int>(p.K);
+  const int32_t* nb = p.nbr + static_cast<int64_t>(n) * K;
+  const float* wn = MODE == FOVI_POOL_GAUSSIAN ? p.w + static_cast<int64_t>(n) * K : nullptr;
+  const int32_t nin = static_cast<int32_t>(p.Nin);
+  int32_t idx[POOL_KF];
+  float w[POOL_KF];
+#pragma unroll
+  for (int j = 0; j < POOL_KF; ++j) {
+    idx[j] = j < K ? nb[j] : -1;
+    if (idx[j] >= nin) idx[j] = -1;
+    w[j] = MODE == FOVI_POOL_GAUSSIAN && j < K ? wn[j] : 0.0f;
+  }
+  const int un = min(PL_U, static_cast<int>(p.C) - static_cast<int>(c0));
+  const InT* xb = static_cast<const InT*>(p.x) + static_cast<int64_t>(b) * p.xs0 + static_cast<int64_t>(c0) * p.xs1;
+  OutT* yb = static_cast<OutT*>(p.y) + static_cast<int64_t>(b) * p.ys0 + static_cast<int64_t>(c0) * p.ys1 +
+             static_cast<int64_t>(n) * p.ys2;
+#pragma unroll 2
+  for (int u = 0; u < un; ++u) {
+    const InT* xp = xb + u * p.xs1;
+    float v[POOL_KF];
+#pragma unroll
+    for (int j = 0; j < POOL_KF; ++j)
+      if (j < K) v[j] = Elem<InT>::load(xp + static_cast<int64_t>(max(idx[j], 0)) * p.xs2);
+    float a = MODE == FOVI_POOL_MAX ? -__builtin_inff() : 0.0f, c = 0.0f;
+#pragma unroll
+    for (int j = 0; j < POOL_KF; ++j) {
+      if (j < K) {
+        const bool use = idx[j] >= 0 && v[j] == v[j];
+        if (MODE == FOVI_POOL_MAX) a = fmaxf(a, use ? v[j] : -__builtin_inff());
+        else if (MODE == FOVI_POOL_GAUSSIAN) a += use ? w[j] : 0.0f;
+        else a += use ? v[j] : 0.0f;
+        if (MODE == FOVI_POOL_AVG) c += use ? 1.0f : 0.0f;
+      }
+    }
+    if (MODE == FOVI_POOL_GAUSSIAN) {
+#pragma unroll
+      for (int j = 0; j < POOL_KF; ++j)
+        if (j < K) {
+          const float t = v[j] * (w[j] / (a + 1e-8f));
+          c += idx[j] >= 0 && v[j] == v[j] ? t : 0.0f;
+        }
+    }
+    PoolAcc st{a, c};
+    Elem<OutT>::store(yb + u * p.ys1, pool_result(st, MODE));
+  }
+}
+
+// Threads along the points of a block (log2) for n points: at most 256, at least 32.
+static int plane_lanes(int64_t n) {
+  int ls = 5;
+  while (ls < 8 && (int64_t(1) << ls) < n) ++ls;
+  return ls;
+}
+
 // any strides: thread = (b, n, c)
 template <typename InT, typename OutT>
 __global__ __launch_bounds__(256) void knnpool_any_kernel(PoolParams p, int64_t total) {
@@ -308,6 +381,26 @@ static void launch_pool(const PoolParams& p, hipStream_t s) {
     return;
   }
   const int64_t total = p.B * p.Nout * p.C;
+  // planes: enough points for a wave's lanes to share a plane row (below 16 the channels are the
+  // better lanes: the last average pooling has one output point)
+  const int64_t cgroups = (p.C + PL_U - 1) / PL_U;
+  const int ls = plane_lanes(p.Nout);
+  const int64_t n_tiles = (p.Nout + (int64_t(1) << ls) - 1) >> ls;
+  const int64_t pblocks = n_tiles * ((p.B * cgroups + (256 >> ls) - 1) / (256 >> ls));
+  if (p.xs2 == 1 && p.K <= POOL_KF && p.Nout >= 16 && p.B * cgroups <= 0x7fffffffLL && pblocks <= 0x7fffffffLL) {
+    const auto args = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(pblocks)), dim3(256), 0, s, p, ls,
+                         static_cast<uint32_t>(n_tiles), static_cast<uint32_t>(cgroups),
+                         static_cast<uint32_t>(p.B * cgroups));
+    };
+    switch (p.mode) {
+      case FOVI_POOL_MAX: args(knnpool_planes_kernel<InT, OutT, FOVI_POOL_MAX>); break;
+      case FOVI_POOL_AVG: args(knnpool_planes_kernel<InT, OutT, FOVI_POOL_AVG>); break;
+      case FOVI_POOL_SUM: args(knnpool_planes_kernel<InT, OutT, FOVI_POOL_SUM>); break;
+      default: args(knnpool_planes_kernel<InT, OutT, FOVI_POOL_GAUSSIAN>); break;
+    }
+    return;
+  }
   const int64_t blocks = std::min<int64_t>((total + 255) / 256, 256 * 64);
   hipLaunchKernelGGL((knnpool_any_kernel<InT, OutT>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, p,
                      total);
@@ -435,9 +528,165 @@ __global__ __launch_bounds__(256) void knnpool_bwd_dx_kernel(PoolBwdParams p, in
   }
 }
 
+// Channel planes (x and dx with unit point stride): thread = (batch row, PL_U consecutive channels,
+// point), lanes along the points, as the forward's planes kernel. The state stays [b, n, c], so
+// a thread reads and writes its PL_U channels' states as one run; dy rows likewise where
+// dy is channels-last (DYR: unit channel stride, 16-byte aligned groups, C % PL_U == 0). The sums
+// run in inverse-list order, as in the kernel above.
+template <typename InT, int MODE>
+__global__ __launch_bounds__(256) void knnpool_bwd_state_planes_kernel(PoolBwdParams p, int ls, uint32_t n_tiles,
+                                                                       uint32_t groups, uint32_t total_groups) {
+  const uint32_t lane = threadIdx.x & ((1u << ls) - 1);
+  const uint32_t n = ((blockIdx.x % n_tiles) << ls) + lane;
+  const uint32_t cg = (blockIdx.x / n_tiles) * (256u >> ls) + (threadIdx.x >> ls);
+  if (n >= static_cast<uint32_t>(p.Nout) || cg >= total_groups) return;
+  const uint32_t b = cg / groups, c0 = (cg % groups) * PL_U;
+  const int K = static_cast<int>(p.K);
+  const int32_t* nb = p.nbr + static_cast<int64_t>(n) * K;
+  const int32_t nin = static_cast<int32_t>(p.Nin);
+  int32_t idx[POOL_KF];
+#pragma unroll
+  for (int j = 0; j < POOL_KF; ++j) {
+    idx[j] = j < K ? nb[j] : -1;
+    if (idx[j] >= nin) idx[j] = -1;
+  }
+  const int un = min(PL_U, static_cast<int>(p.C) - static_cast<int>(c0));
+  const InT* xb = static_cast<const InT*>(p.x) + static_cast<int64_t>(b) * p.xs0 + static_cast<int64_t>(c0) * p.xs1;
+  float* st = p.state + (static_cast<int64_t>(b) * p.Nout + n) * p.C + c0;
+#pragma unroll 2
+  for (int u = 0; u < un; ++u) {
+    const InT* xp = xb + u * p.xs1;
+    float v[POOL_KF];
+#pragma unroll
+    for (int j = 0; j < POOL_KF; ++j)
+      if (j < K) v[j] = Elem<InT>::load(xp + static_cast<int64_t>(max(idx[j], 0)) * p.xs2);
+    float best = -__builtin_inff(), sum = 0.0f;
+    int arg = 0;
+#pragma unroll
+    for (int j = 0; j < POOL_KF; ++j) {
+      if (j < K) {
+        const bool use = idx[j] >= 0 && v[j] == v[j];
+        if (MODE == FOVI_POOL_MAX) {
+          const float m = use ? v[j] : -__builtin_inff();
+          if (j == 0 || m > best) { best = m; arg = j; }      // first position of the maximum
+        } else if (use) {
+          sum += MODE == FOVI_POOL_GAUSSIAN ? p.w[static_cast<int64_t>(n) * K + j] : 1.0f;
+        }
+      }
+    }
+    st[u] = MODE == FOVI_POOL_MAX ? static_cast<float>(arg) : (MODE == FOVI_POOL_GAUSSIAN ? sum + 1e-8f : sum);
+  }
+}
+
+template <typename InT, typename GT, typename DT, int MODE, bool DYR>
+__global__ __launch_bounds__(256) void knnpool_bwd_dx_planes_kernel(PoolBwdParams p, int ls, uint32_t n_tiles,
+                                                                    uint32_t groups, uint32_t total_groups) {
+  const uint32_t lane = threadIdx.x & ((1u << ls) - 1);
+  const uint32_t i = ((blockIdx.x % n_tiles) << ls) + lane;
+  const uint32_t cg = (blockIdx.x / n_tiles) * (256u >> ls) + (threadIdx.x >> ls);
+  if (i >= static_cast<uint32_t>(p.Nin) || cg >= total_groups) return;
+  const uint32_t b = cg / groups, c0 = (cg % groups) * PL_U;
+  const int un = min(PL_U, static_cast<int>(p.C) - static_cast<int>(c0));
+  const uint32_t K = static_cast<uint32_t>(p.K);
+  const InT* xb = static_cast<const InT*>(p.x) + static_cast<int64_t>(b) * p.xs0 + static_cast<int64_t>(c0) * p.xs1 +
+                  static_cast<int64_t>(i) * p.xs2;
+  const GT* dyb = static_cast<const GT*>(p.dy) + static_cast<int64_t>(b) * p.ds0 + static_cast<int64_t>(c0) * p.ds1;
+  const float* stb = p.state + static_cast<int64_t>(b) * p.Nout * p.C + c0;
+  float acc[PL_U];
+#pragma unroll
+  for (int u = 0; u < PL_U; ++u) acc[u] = 0.0f;
+  const int32_t q1 = p.inv_ptr[i + 1];
+  for (int32_t q = p.inv_ptr[i]; q < q1; ++q) {
+    const uint32_t e = static_cast<uint32_t>(p.inv[q]);
+    const uint32_t n = e / K, j = e - n * K;
+    const float w = MODE == FOVI_POOL_GAUSSIAN ? p.w[e] : 0.0f;
+    float g[PL_U], st[PL_U];
+    if constexpr (DYR) {
+      constexpr int NV = Vec16<GT>::N;
+#pragma unroll
+      for (int h = 0; h < PL_U / NV; ++h) {
+        float t[NV];
+        Vec16<GT>::load(dyb + static_cast<int64_t>(n) * p.ds2 + h * NV, t);
+#pragma unroll
+        for (int u = 0; u < NV; ++u) g[h * NV + u] = t[u];
+      }
+      if (MODE != FOVI_POOL_SUM) {
+        const f32x4* s4 = reinterpret_cast<const f32x4*>(stb + static_cast<int64_t>(n) * p.C);
+        const f32x4 s0 = s4[0], s1 = s4[1];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { st[u] = s0[u]; st[4 + u] = s1[u]; }
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < PL_U; ++u) {
+        const int uc = u < un ? u : 0;
+        g[u] = Elem<GT>::load(dyb + uc * p.ds1 + static_cast<int64_t>(n) * p.ds2);
+        if (MODE != FOVI_POOL_SUM) st[u] = stb[static_cast<int64_t>(n) * p.C + uc];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PL_U; ++u) {
+      switch (MODE) {
+        case FOVI_POOL_MAX: if (st[u] == static_cast<float>(j)) acc[u] += g[u]; break;
+        case FOVI_POOL_AVG: acc[u] += g[u] / st[u]; break;
+        case FOVI_POOL_SUM: acc[u] += g[u]; break;
+        default: acc[u] += g[u] * (w / st[u]); break;
+      }
+    }
+  }
+  DT* dxb = static_cast<DT*>(p.dx) + static_cast<int64_t>(b) * p.gs0 + static_cast<int64_t>(c0) * p.gs1 +
+            static_cast<int64_t>(i) * p.gs2;
+#pragma unroll
+  for (int u = 0; u < PL_U; ++u)
+    if (u < un) {
+      const float xv = Elem<InT>::load(xb + u * p.xs1);
+      Elem<DT>::store(dxb + u * p.gs1, xv == xv ? acc[u] : 0.0f);      // a NaN feature carries none
+    }
+}
+
+template <typename InT, typename GT, int MODE>
+static void launch_pool_bwd_planes(const PoolBwdParams& p, bool dx_f32, int64_t cgroups, hipStream_t s) {
+  const uint32_t groups = static_cast<uint32_t>(cgroups), total = static_cast<uint32_t>(p.B * cgroups);
+  const auto tiles = [](int64_t n, int ls) { return static_cast<uint32_t>((n + (int64_t(1) << ls) - 1) >> ls); };
+  const auto grid = [&](uint32_t nt, int ls) {
+    return dim3(static_cast<unsigned>(nt * ((total + (256u >> ls) - 1) / (256u >> ls))));
+  };
+  if (MODE != FOVI_POOL_SUM && p.Nout > 0) {
+    const int ls = plane_lanes(p.Nout);
+    hipLaunchKernelGGL((knnpool_bwd_state_planes_kernel<InT, MODE>), grid(tiles(p.Nout, ls), ls), dim3(256), 0, s, p,
+                       ls, tiles(p.Nout, ls), groups, total);
+  }
+  const int ls = plane_lanes(p.Nin);
+  const uint32_t nt = tiles(p.Nin, ls);
+  const int64_t al = 16 / static_cast<int64_t>(sizeof(GT));
+  const bool rows = p.ds1 == 1 && p.C % PL_U == 0 && p.ds0 % al == 0 && p.ds2 % al == 0 &&
+                    (reinterpret_cast<uintptr_t>(p.dy) | reinterpret_cast<uintptr_t>(p.state)) % 16 == 0;
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid(nt, ls), dim3(256), 0, s, p, ls, nt, groups, total);
+  };
+  if (dx_f32) {
+    if (rows) go(knnpool_bwd_dx_planes_kernel<InT, GT, float, MODE, true>);
+    else go(knnpool_bwd_dx_planes_kernel<InT, GT, float, MODE, false>);
+  } else {
+    if (rows) go(knnpool_bwd_dx_planes_kernel<InT, GT, uint16_t, MODE, true>);
+    else go(knnpool_bwd_dx_planes_kernel<InT, GT, uint16_t, MODE, false>);
+  }
+}
+
 template <typename InT, typename GT>
 static void launch_pool_bwd(const PoolBwdParams& p, bool dx_f32, hipStream_t s) {
   const int64_t n1 = p.B * p.Nout * p.C, n2 = p.B * p.Nin * p.C;
+  const int64_t cgroups = (p.C + PL_U - 1) / PL_U;
+  if (p.xs2 == 1 && p.gs2 == 1 && p.K <= POOL_KF && p.Nin >= 16 && p.Nout > 0 && n2 > 0 && p.Nout * p.K < 0x7fffffffLL &&
+      p.B * cgroups * ((p.Nin + 31) / 32) <= 0x3fffffffLL && p.B * cgroups * ((p.Nout + 31) / 32) <= 0x3fffffffLL) {
+    switch (p.mode) {
+      case FOVI_POOL_MAX: launch_pool_bwd_planes<InT, GT, FOVI_POOL_MAX>(p, dx_f32, cgroups, s); break;
+      case FOVI_POOL_AVG: launch_pool_bwd_planes<InT, GT, FOVI_POOL_AVG>(p, dx_f32, cgroups, s); break;
+      case FOVI_POOL_SUM: launch_pool_bwd_planes<InT, GT, FOVI_POOL_SUM>(p, dx_f32, cgroups, s); break;
+      default: launch_pool_bwd_planes<InT, GT, FOVI_POOL_GAUSSIAN>(p, dx_f32, cgroups, s); break;
+    }
+    return;
+  }
   auto grid = [](int64_t n) { return dim3(static_cast<unsigned>(std::min<int64_t>((n + 255) / 256, 256 * 64))); };
   if (p.mode != FOVI_POOL_SUM && n1 > 0)
     hipLaunchKernelGGL((knnpool_bwd_state_kernel<InT>), grid(n1), dim3(256), 0, s, p, n1);
