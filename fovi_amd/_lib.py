@@ -14,7 +14,7 @@ import torch
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libfovi_hip.so")
 
-ABI_VERSION = 34
+ABI_VERSION = 35
 F32, BF16, F8E4M3 = 0, 1, 2
 NEAREST, BILINEAR = 0, 1
 PAD_ZEROS, PAD_BORDER = 0, 1
@@ -31,7 +31,8 @@ EXPORTED = ("fovi_abi_version", "fovi_last_error", "fovi_sampler_fwd", "fovi_knn
             "fovi_knn_logpolar_candidates", "fovi_knn_select", "fovi_knn_euclid_candidates", "fovi_local_rf_slots", "fovi_knnconv_dw_workspace_bytes",
             "fovi_knnconv_dw", "fovi_knnpool_bwd", "fovi_knnconv_last_path",
             "fovi_knnconv_fwd_noalloc", "fovi_knnconv_wide_tiles", "fovi_knnconv_weight_img_elems",
-            "fovi_knnconv_pack_weight_img", "fovi_knnconv_img_tables")
+            "fovi_knnconv_pack_weight_img", "fovi_knnconv_img_tables", "fovi_knnconv_dw_few",
+            "fovi_knnconv_dw_few_workspace_bytes")
 
 
 class SamplerArgs(C.Structure):
@@ -193,6 +194,18 @@ class KnnConvDwArgs(C.Structure):
     ]
 
 
+class KnnConvDwFewArgs(C.Structure):
+    _fields_ = [
+        ("x", C.c_void_p), ("x_dtype", C.c_int32), ("reserved0", C.c_int32), ("x_stride", C.c_int64 * 3),
+        ("dy", C.c_void_p), ("dy_stride", C.c_int64 * 3),
+        ("batch", C.c_int64), ("c_in", C.c_int64), ("c_out", C.c_int64), ("n_in", C.c_int64),
+        ("n_out", C.c_int64), ("k", C.c_int64), ("n_ref", C.c_int64),
+        ("slot_ptr", C.c_void_p), ("nbr_sorted", C.c_void_p),
+        ("workspace", C.c_void_p), ("workspace_bytes", C.c_int64),
+        ("dw", C.c_void_p),
+    ]
+
+
 _lib = None
 
 
@@ -250,6 +263,10 @@ def load(path: str = LIB_PATH):
     lib.fovi_knnconv_dw_workspace_bytes.restype = C.c_int64
     lib.fovi_knnconv_dw.argtypes = [C.POINTER(KnnConvDwArgs), C.c_void_p]
     lib.fovi_knnconv_dw.restype = C.c_int
+    lib.fovi_knnconv_dw_few_workspace_bytes.argtypes = [C.c_int64] * 6 + [C.c_int32]
+    lib.fovi_knnconv_dw_few_workspace_bytes.restype = C.c_int64
+    lib.fovi_knnconv_dw_few.argtypes = [C.POINTER(KnnConvDwFewArgs), C.c_void_p]
+    lib.fovi_knnconv_dw_few.restype = C.c_int
     lib.fovi_knnpool_bwd.argtypes = [C.POINTER(KnnPoolBwdArgs), C.c_void_p]
     lib.fovi_knnpool_bwd.restype = C.c_int
     lib.fovi_knnconv_wide_tiles.argtypes = [C.c_int64] + [C.c_int32] * 5 + [C.POINTER(C.c_int64)]

@@ -899,13 +899,18 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         bsz, c, n_in = x.shape
         n_out, v, c_out = self.out_coords.shape[0], self.ref_coords.shape[0], self.out_channels
         dt = x.dtype
+        dw_few = self._dw_few(x, dy) if need_w and self.dw_fused and dy.dtype == torch.bfloat16 and c <= 8 else None
+        if dw_few is not None and not need_x:
+            return None, dw_few.to(weight.dtype)
         dy = dy.to(dt)
         if dy.stride(1) != 1:       # channels-last once, for every kernel below
             dy = dy.transpose(1, 2).contiguous().transpose(1, 2)
         lib = _lib.load()
         stream = _lib.stream_handle(x.device)
         dx = dw = None
-        if need_w and self.dw_fused and self._dw_fused_ok(x, dt):
+        if dw_few is not None:
+            dw = dw_few.to(weight.dtype)
+        elif need_w and self.dw_fused and self._dw_fused_ok(x, dt):
             dw = self._dw_fused(x, dy).to(weight.dtype)
         elif need_w:
             dy2 = dy.permute(0, 2, 1).reshape(bsz * n_out, c_out)
@@ -944,6 +949,27 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         return (dt == torch.bfloat16 and self.in_channels % 8 == 0 and self.out_channels % 8 == 0
                 and x.stride(1) == 1 and x.stride(2) % 8 == 0 and x.stride(0) % 8 == 0
                 and x.data_ptr() % 16 == 0)
+
+    def _dw_few(self, x, dy):
+        """``dW`` (fp32, reference layout) of a layer with at most 8 input channels from a bf16 ``dy`` of
+        any layout (``fovi_knnconv_dw_few``), or None for sizes it does not take."""
+        bsz, c, n_in = x.shape
+        n_out, v, c_out = self.out_coords.shape[0], self.ref_coords.shape[0], self.out_channels
+        lib = _lib.load()
+        nbytes = lib.fovi_knnconv_dw_few_workspace_bytes(bsz, c, c_out, n_in, n_out, v, _lib.dtype_code(x.dtype))
+        if nbytes < 0 or self._k > 32767:
+            return None
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+        dw = torch.empty(c_out, c * v, dtype=torch.float32, device=x.device)
+        a = _lib.KnnConvDwFewArgs()
+        a.x = x.data_ptr(); a.x_dtype = _lib.dtype_code(x.dtype); a.x_stride[:] = list(x.stride())
+        a.dy = dy.data_ptr(); a.dy_stride[:] = list(dy.stride())
+        a.batch, a.c_in, a.c_out, a.n_in, a.n_out, a.k, a.n_ref = bsz, c, c_out, n_in, n_out, self._k, v
+        a.slot_ptr = self.slot_ptr.data_ptr(); a.nbr_sorted = self.nbr_sorted.data_ptr()
+        a.workspace = ws.data_ptr(); a.workspace_bytes = nbytes
+        a.dw = dw.data_ptr()
+        _lib.check(lib.fovi_knnconv_dw_few(a, _lib.stream_handle(x.device)), "fovi_knnconv_dw_few")
+        return dw
 
     def _dw_fused(self, x, dy):
         """``dW`` (fp32, reference layout) by ``fovi_knnconv_dw``: per slot a GEMM over its

@@ -1,0 +1,352 @@
+// Weight gradient of few-channel kNN-conv layers (c_in <= 8) from a bf16 output gradient:
+// dW[o, c * V + v] = sum over images b and the (output n, input i) pairs of slot v of
+// dy[b, n, o] * x[b, i, c], x fp32 or bf16.
+//
+// The images are the reduction index of the matrix instructions. A first pass lays both operands
+// out with the images adjacent (dyT[n][o][b], xT[i][c][b], bf16, images padded with zeros to
+// 16), so that a lane loads its 8 images of one row or column with one 16-byte load and nothing
+// passes through LDS. fp32 x is split into three bf16 parts by truncation (8 + 8 + 8 significant
+// bits: exact), each multiplied with dy: the products are exact, the sums fp32, as in an fp32
+// product.
+// A wave owns all rows o of a tile of up to 96 and two blocks of 32 columns, 32 / c_in slots x
+// c_in channels each; for every point of its range it reads the slots' neighbour lists, one
+// neighbour of every slot per round (a slot without one reads a zero row), and skips a block none
+// of whose slots has a neighbour (not with a non-finite dy: its product with an empty slot's zero
+// is NaN). Partial tiles per point range go to a workspace and are
+// added in range order.
+// 128 images, 3 -> 96 channels, 4085 -> 964 points, k = 121 in V = 484 slots, x fp32: the slot-sum
+// matrix (717 MB) and an fp32 GEMM over it took 650 + 643 us.
+#include <type_traits>
+
+#include "common.h"
+
+namespace fovi {
+namespace {
+
+typedef uint32_t u32x4f __attribute__((ext_vector_type(4)));
+
+constexpr int DF_CT = 2;                 // column blocks per wave
+constexpr int DF_WAVES = 4;
+
+// ---- operands with the images adjacent ------------------------------------------------------
+// out[(fast * of + slow * os) * bp + b], planes of `plane` elements apart for the parts; a block
+// takes 64 fast indices of one slow index and 64 images through LDS: reads run along the fast
+// dimension of the input, writes along the images.
+struct LayoutParams {
+  const void* in;
+  int64_t B, F, S, sb, sf, ss;           // images, fast and slow counts, their element strides
+  uint16_t* out;
+  int64_t of, os, bp, plane;
+  int32_t* flag;                         // set if a value is not finite (or NULL)
+};
+
+template <typename InT, int NS>
+__global__ __launch_bounds__(256) void images_adjacent_kernel(LayoutParams p, uint32_t f_tiles, uint32_t b_tiles) {
+  typedef typename std::conditional<std::is_same<InT, float>::value, float, uint16_t>::type T;
+  __shared__ T tile[64][65];
+  const uint32_t ft = blockIdx.x % f_tiles, rest = blockIdx.x / f_tiles;
+  const int64_t f0 = static_cast<int64_t>(ft) * 64, b0 = static_cast<int64_t>(rest % b_tiles) * 64;
+  const int64_t s = rest / b_tiles;
+  const T* in = static_cast<const T*>(p.in) + s * p.ss;
+  for (int k = threadIdx.x >> 6; k < 64; k += 4) {
+    const int64_t f = f0 + (threadIdx.x & 63), b = b0 + k;
+    tile[k][threadIdx.x & 63] = f < p.F && b < p.B ? in[b * p.sb + f * p.sf] : T(0);
+  }
+  __syncthreads();
+  // 32 pairs of images x 8 fast indices per pass: 4-byte stores
+  for (int k = threadIdx.x >> 5; k < 64; k += 8) {
+    const int64_t f = f0 + k, b = b0 + 2 * (threadIdx.x & 31);
+    if (f >= p.F || b >= p.bp) continue;
+    uint16_t part[2][NS];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const T v = tile[2 * (threadIdx.x & 31) + u][k];
+      if constexpr (NS == 1) {
+        part[u][0] = v;
+        if (p.flag && (v & 0x7f80u) == 0x7f80u) *p.flag = 1;
+      } else {
+        // by truncation: the parts add up to v exactly; a non-finite v is its own first part
+        const uint32_t bits = __float_as_uint(v);
+        const float h = __uint_as_float(bits & 0xffff0000u);
+        const bool fin = (bits & 0x7f800000u) != 0x7f800000u;
+        const float r1 = fin ? v - h : 0.0f;
+        const float m = __uint_as_float(__float_as_uint(r1) & 0xffff0000u);
+        part[u][0] = static_cast<uint16_t>(bits >> 16);
+        if (!fin && (bits & 0x007fffffu) && !(bits & 0x007f0000u)) part[u][0] |= 1;   // NaN stays NaN
+        part[u][1] = static_cast<uint16_t>(__float_as_uint(m) >> 16);
+        part[u][NS - 1] = static_cast<uint16_t>(__float_as_uint(r1 - m) >> 16);
+      }
+    }
+    uint16_t* o = p.out + (f * p.of + s * p.os) * p.bp + b;
+#pragma unroll
+    for (int q = 0; q < NS; ++q)
+      *reinterpret_cast<uint32_t*>(o + q * p.plane) = part[0][q] | static_cast<uint32_t>(part[1][q]) << 16;
+  }
+}
+
+__global__ __launch_bounds__(256) void zero_rows_kernel(uint16_t* out, int64_t count, int64_t plane, int ns,
+                                                        int32_t* flag) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i == 0) *flag = 0;
+  if (i < count)
+    for (int q = 0; q < ns; ++q) out[q * plane + i] = 0;
+}
+
+// ---- the products ------------------------------------------------------------------------------
+struct DwFewParams {
+  const uint16_t* dyt;                   // [n_out][c_out][bp]
+  const uint16_t* xt;                    // [parts][n_in + 1][c_in][bp], row n_in zero
+  int64_t plane;
+  int C, Cout, Nin, Nout, V, K, bp;
+  int slots;                             // slots per column block: 32 / c_in
+  int n_ct, per;                         // column tiles (of DF_CT blocks), points per range
+  const int32_t* slot_ptr;
+  const int32_t* nbr;
+  const int32_t* flag;                   // dy holds a non-finite value
+  float* part;                           // [ranges][o tiles][n_ct][MB * 32][DF_CT * 32]
+};
+
+template <int MB, int NS>
+__global__ __launch_bounds__(DF_WAVES * 64, 2) void knnconv_dw_few_kernel(DwFewParams p, int ct_groups) {
+  const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ct = static_cast<int>(blockIdx.x % ct_groups) * DF_WAVES + wave;
+  const int range = blockIdx.x / ct_groups;
+  const int o0 = blockIdx.y * MB * 32;
+  if (ct >= p.n_ct) return;              // no barrier follows
+  const int n0 = range * p.per, n1 = min(p.Nout, n0 + p.per);
+
+  // this lane's column of each block: slot v[b], channel c (columns past the slots: none)
+  int v[DF_CT];
+  const int c = l32 % p.C;
+#pragma unroll
+  for (int b = 0; b < DF_CT; ++b) {
+    const int s = l32 / p.C;
+    v[b] = s < p.slots ? (ct * DF_CT + b) * p.slots + s : p.V;
+    if (v[b] >= p.V) v[b] = -1;
+  }
+  uint32_t oa[MB];                       // row offsets of dyT within a point
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+    const int o = min(o0 + m * 32 + l32, p.Cout - 1);
+    oa[m] = static_cast<uint32_t>(o) * p.bp + 8 * h;
+  }
+
+  f32x16 acc[MB][DF_CT];
+#pragma unroll
+  for (int m = 0; m < MB; ++m)
+#pragma unroll
+    for (int b = 0; b < DF_CT; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[m][b][r] = 0.0f;
+
+  auto words = [&](int n, int (&w)[DF_CT]) {
+#pragma unroll
+    for (int b = 0; b < DF_CT; ++b) w[b] = n < n1 && v[b] >= 0 ? p.slot_ptr[static_cast<int64_t>(n) * p.V + v[b]] : 0;
+  };
+  auto row = [&](int n, int w, int r) {  // the slot's r-th neighbour, or the zero row
+    return r < (w & 0xffff) ? p.nbr[static_cast<int64_t>(n) * p.K + (w >> 16) + r] : p.Nin;
+  };
+  const bool every = *p.flag != 0;
+  int w[DF_CT], wn[DF_CT], i0[DF_CT];
+  words(n0, w);
+#pragma unroll
+  for (int b = 0; b < DF_CT; ++b) i0[b] = n0 < n1 ? row(n0, w[b], 0) : p.Nin;
+  words(n0 + 1, wn);
+  for (int n = n0; n < n1; ++n) {
+    int inx[DF_CT], wnn[DF_CT];          // the next point's first neighbours, the one after's words
+#pragma unroll
+    for (int b = 0; b < DF_CT; ++b) inx[b] = n + 1 < n1 ? row(n + 1, wn[b], 0) : p.Nin;
+    words(n + 2, wnn);
+    const uint16_t* dn = p.dyt + static_cast<int64_t>(n) * p.Cout * p.bp;
+    for (int r = 0;; ++r) {
+      bool on[DF_CT];
+      const uint16_t* xb[DF_CT];
+      bool any = false;
+#pragma unroll
+      for (int b = 0; b < DF_CT; ++b) {
+        on[b] = __builtin_amdgcn_ballot_w64((w[b] & 0xffff) > r) != 0 || (every && r == 0);
+        any |= on[b];
+        const int i = r == 0 ? i0[b] : row(n, w[b], r);
+        xb[b] = p.xt + (static_cast<int64_t>(i) * p.C + c) * p.bp + 8 * h;
+      }
+      if (!any) break;
+      // the blocks of this round (uniform): one loop each, so that no product is conditional
+      auto run = [&](auto first, auto last) __attribute__((always_inline)) {
+        constexpr int B0 = decltype(first)::value, B1 = decltype(last)::value;
+#pragma unroll 1
+        for (int k = 0; k < p.bp; k += 16) {
+          bf16x8 a[MB], x[B1 - B0][NS];
+#pragma unroll
+          for (int m = 0; m < MB; ++m) a[m] = *reinterpret_cast<const bf16x8*>(dn + oa[m] + k);
+#pragma unroll
+          for (int b = B0; b < B1; ++b)
+#pragma unroll
+            for (int q = 0; q < NS; ++q) x[b - B0][q] = *reinterpret_cast<const bf16x8*>(xb[b] + q * p.plane + k);
+#pragma unroll
+          for (int b = B0; b < B1; ++b)
+#pragma unroll
+            for (int q = NS - 1; q >= 0; --q)          // small parts first
+#pragma unroll
+              for (int m = 0; m < MB; ++m)
+                acc[m][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[m], x[b - B0][q], acc[m][b], 0, 0, 0);
+        }
+      };
+      typedef std::integral_constant<int, 0> I0;
+      typedef std::integral_constant<int, 1> I1;
+      typedef std::integral_constant<int, 2> I2;
+      if (on[0] && on[1]) run(I0(), I2());
+      else if (on[0]) run(I0(), I1());
+      else run(I1(), I2());
+    }
+#pragma unroll
+    for (int b = 0; b < DF_CT; ++b) { w[b] = wn[b]; wn[b] = wnn[b]; i0[b] = inx[b]; }
+  }
+  float* out = p.part + ((static_cast<int64_t>(range) * gridDim.y + blockIdx.y) * p.n_ct + ct) * (MB * 32 * DF_CT * 32);
+#pragma unroll
+  for (int m = 0; m < MB; ++m)
+#pragma unroll
+    for (int b = 0; b < DF_CT; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        out[(m * 32 + 8 * (r >> 2) + 4 * h + (r & 3)) * (DF_CT * 32) + b * 32 + l32] = acc[m][b][r];
+}
+
+__global__ __launch_bounds__(256) void knnconv_dw_few_reduce_kernel(DwFewParams p, int mb, int ranges, int o_tiles,
+                                                                    float* dw) {
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (t >= static_cast<int64_t>(p.Cout) * p.C * p.V) return;
+  const int v = static_cast<int>(t % p.V);
+  const int c = static_cast<int>((t / p.V) % p.C), o = static_cast<int>(t / (static_cast<int64_t>(p.V) * p.C));
+  const int blk = v / p.slots, col = (v % p.slots) * p.C + c;
+  const int rows = mb * 32;
+  const float* src = p.part + (static_cast<int64_t>(o / rows) * p.n_ct + blk / DF_CT) * (rows * DF_CT * 32) +
+                     (o % rows) * (DF_CT * 32) + (blk % DF_CT) * 32 + col;
+  const int64_t stride = static_cast<int64_t>(o_tiles) * p.n_ct * rows * DF_CT * 32;
+  float sum = 0.0f;
+  int s = 0;
+  for (; s + 8 <= ranges; s += 8) {
+    float x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = src[(s + u) * stride];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) sum += x[u];
+  }
+  for (; s < ranges; ++s) sum += src[s * stride];
+  dw[t] = sum;
+}
+
+struct FewPlan {
+  int64_t bp, dyt, xt, part;             // images padded; elements of dyT, xT (a part), partials
+  int parts, slots, n_ct, mb, o_tiles, ranges, per;
+};
+
+bool few_plan(int64_t B, int64_t C, int64_t Cout, int64_t Nin, int64_t Nout, int64_t V, int x_dtype, FewPlan& f) {
+  if (B < 1 || C < 1 || C > 8 || Cout < 1 || Nin < 1 || Nout < 1 || V < 1 || (x_dtype != FOVI_F32 && x_dtype != FOVI_BF16))
+    return false;
+  constexpr int64_t lim = int64_t(1) << 31;
+  f.bp = (B + 15) / 16 * 16;
+  if (f.bp >= (1 << 20) || Cout >= (1 << 20) || Nin >= lim - 1 || Nout >= lim || V >= (1 << 20) || Cout * f.bp >= lim)
+    return false;
+  f.parts = x_dtype == FOVI_F32 ? 3 : 1;
+  f.slots = static_cast<int>(32 / C);
+  const int64_t blocks = (V + f.slots - 1) / f.slots;
+  f.n_ct = static_cast<int>((blocks + DF_CT - 1) / DF_CT);
+  // tiles of up to 96 rows (128 rows x 2 blocks spill their accumulators), as even as they come
+  const int64_t row_blocks = (Cout + 31) / 32;
+  f.o_tiles = static_cast<int>((row_blocks + 2) / 3);
+  f.mb = static_cast<int>((row_blocks + f.o_tiles - 1) / f.o_tiles);
+  // point ranges: about 3072 waves in all (three per SIMD), each range at least one point
+  const int64_t tiles = static_cast<int64_t>(f.n_ct) * f.o_tiles;
+  int64_t ranges = (3072 + tiles - 1) / tiles;
+  if (ranges > Nout) ranges = Nout;
+  const int64_t per = (Nout + ranges - 1) / ranges;
+  f.per = static_cast<int>(per);
+  f.ranges = static_cast<int>((Nout + per - 1) / per);
+  f.dyt = (Nout * Cout * f.bp + 63) / 64 * 64;
+  f.xt = ((Nin + 1) * C * f.bp + 63) / 64 * 64;
+  f.part = static_cast<int64_t>(f.ranges) * tiles * f.mb * 32 * DF_CT * 32;
+  return true;
+}
+
+template <typename InT, int NS>
+int lay_out(const void* in, int64_t B, int64_t C, int64_t N, const int64_t* st, uint16_t* out, int64_t bp, int64_t plane,
+            int32_t* flag, hipStream_t s) {
+  LayoutParams p;
+  p.in = in; p.B = B; p.sb = st[0]; p.out = out; p.bp = bp; p.plane = plane; p.flag = flag;
+  const bool rows = st[1] == 1 && C > 1;         // channels adjacent: they are the fast dimension
+  p.F = rows ? C : N; p.S = rows ? N : C;
+  p.sf = rows ? st[1] : st[2]; p.ss = rows ? st[2] : st[1];
+  p.of = rows ? 1 : C; p.os = rows ? C : 1;      // row n * C + c
+  const int64_t ft = (p.F + 63) / 64, bt = (bp + 63) / 64;
+  if (ft * bt * p.S > 0x7fffffffLL) { set_error("fovi_knnconv_dw_few: too large"); return 1; }
+  hipLaunchKernelGGL((images_adjacent_kernel<InT, NS>), dim3(static_cast<unsigned>(ft * bt * p.S)), dim3(256), 0, s, p,
+                     static_cast<uint32_t>(ft), static_cast<uint32_t>(bt));
+  return check_launch("fovi_knnconv_dw_few(layout)");
+}
+
+template <int NS>
+int launch_few(const DwFewParams& p, const FewPlan& f, hipStream_t s) {
+  const int groups = (f.n_ct + DF_WAVES - 1) / DF_WAVES;
+  const dim3 grid(static_cast<unsigned>(static_cast<int64_t>(groups) * f.ranges), static_cast<unsigned>(f.o_tiles));
+  const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(DF_WAVES * 64), 0, s, p, groups); };
+  if (f.mb == 1) go(knnconv_dw_few_kernel<1, NS>);
+  else if (f.mb == 2) go(knnconv_dw_few_kernel<2, NS>);
+  else go(knnconv_dw_few_kernel<3, NS>);
+  return check_launch("fovi_knnconv_dw_few");
+}
+
+}  // namespace
+}  // namespace fovi
+
+extern "C" int64_t fovi_knnconv_dw_few_workspace_bytes(int64_t batch, int64_t c_in, int64_t c_out, int64_t n_in,
+                                                       int64_t n_out, int64_t n_ref, int32_t x_dtype) {
+  fovi::FewPlan f;
+  if (!fovi::few_plan(batch, c_in, c_out, n_in, n_out, n_ref, x_dtype, f)) return -1;
+  return (f.dyt + f.parts * f.xt) * 2 + f.part * 4 + 16;
+}
+
+extern "C" int fovi_knnconv_dw_few(const fovi_knnconv_dw_few_args* a, void* stream) {
+  using namespace fovi;
+  clear_error();
+  if (!a || !a->x || !a->dy || !a->slot_ptr || !a->nbr_sorted || !a->workspace || !a->dw) {
+    set_error("fovi_knnconv_dw_few: null pointer");
+    return 1;
+  }
+  FewPlan f;
+  if (a->k < 1 || a->k > 32767 || !few_plan(a->batch, a->c_in, a->c_out, a->n_in, a->n_out, a->n_ref, a->x_dtype, f)) {
+    set_error("fovi_knnconv_dw_few: bad sizes (1 to 8 input channels, F32 or BF16 input)");
+    return 1;
+  }
+  const int64_t need = (f.dyt + f.parts * f.xt) * 2 + f.part * 4 + 16;
+  if (a->workspace_bytes < need || reinterpret_cast<uintptr_t>(a->workspace) % 16 != 0) {
+    set_error("fovi_knnconv_dw_few: workspace %lld bytes (16-byte aligned), need %lld", (long long)a->workspace_bytes,
+              (long long)need);
+    return 1;
+  }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  DwFewParams p;
+  float* part = static_cast<float*>(a->workspace);             // a multiple of 128 bytes
+  uint16_t* dyt = reinterpret_cast<uint16_t*>(part + f.part);
+  uint16_t* xt = dyt + f.dyt;
+  int32_t* flag = reinterpret_cast<int32_t*>(xt + f.parts * f.xt);
+  const int64_t zero = a->c_in * f.bp;
+  hipLaunchKernelGGL(zero_rows_kernel, dim3(static_cast<unsigned>((zero + 255) / 256)), dim3(256), 0, s,
+                     xt + a->n_in * zero, zero, f.xt, f.parts, flag);
+  if (check_launch("fovi_knnconv_dw_few(zero row)")) return 1;
+  if (lay_out<uint16_t, 1>(a->dy, a->batch, a->c_out, a->n_out, a->dy_stride, dyt, f.bp, 0, flag, s)) return 1;
+  if (a->x_dtype == FOVI_F32 ? lay_out<float, 3>(a->x, a->batch, a->c_in, a->n_in, a->x_stride, xt, f.bp, f.xt, nullptr, s)
+                             : lay_out<uint16_t, 1>(a->x, a->batch, a->c_in, a->n_in, a->x_stride, xt, f.bp, f.xt,
+                                                    nullptr, s))
+    return 1;
+  p.dyt = dyt; p.xt = xt; p.plane = f.xt;
+  p.C = static_cast<int>(a->c_in); p.Cout = static_cast<int>(a->c_out); p.Nin = static_cast<int>(a->n_in);
+  p.Nout = static_cast<int>(a->n_out); p.V = static_cast<int>(a->n_ref); p.K = static_cast<int>(a->k);
+  p.bp = static_cast<int>(f.bp); p.slots = f.slots; p.n_ct = f.n_ct; p.per = f.per;
+  p.slot_ptr = a->slot_ptr; p.nbr = a->nbr_sorted; p.flag = flag; p.part = part;
+  if (f.parts == 3 ? launch_few<3>(p, f, s) : launch_few<1>(p, f, s)) return 1;
+  const int64_t n = a->c_out * a->c_in * a->n_ref;
+  hipLaunchKernelGGL(knnconv_dw_few_reduce_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s, p, f.mb,
+                     f.ranges, f.o_tiles, a->dw);
+  return check_launch("fovi_knnconv_dw_few(reduce)");
+}

@@ -23,7 +23,7 @@
 extern "C" {
 #endif
 
-#define FOVI_ABI_VERSION 34
+#define FOVI_ABI_VERSION 35
 
 enum fovi_dtype { FOVI_F32 = 0, FOVI_BF16 = 1, FOVI_F8E4M3 = 2 };
 enum fovi_interp { FOVI_NEAREST = 0, FOVI_BILINEAR = 1 };
@@ -716,6 +716,32 @@ typedef struct fovi_knnconv_dw_args {
 int64_t fovi_knnconv_dw_workspace_bytes(int64_t batch, int64_t images_per_group, int64_t n_chunks, int64_t c_in,
                                         int64_t c_out, int64_t n_ref);
 int fovi_knnconv_dw(const fovi_knnconv_dw_args* args, void* stream);
+
+/*
+ * The same gradient for layers with 1 to 8 input channels, from a bf16 dy and an F32 or BF16 x of
+ * any element strides [batch, channel, point]; fp32 x enters as three bf16 parts that add up to it
+ * exactly. slot_ptr [n_out, n_ref] and nbr_sorted [n_out, k] are the forward's tables. The
+ * workspace (fovi_knnconv_dw_few_workspace_bytes, -1 for sizes it does not take; 16-byte
+ * aligned) holds both operands with the images adjacent and the partial sums.
+ */
+typedef struct fovi_knnconv_dw_few_args {
+  const void* x;
+  int32_t x_dtype;
+  int32_t reserved0;
+  int64_t x_stride[3];
+  const void* dy;             /* bf16 */
+  int64_t dy_stride[3];
+  int64_t batch, c_in, c_out, n_in, n_out, k, n_ref;
+  const int32_t* slot_ptr;
+  const int32_t* nbr_sorted;
+  void* workspace;
+  int64_t workspace_bytes;
+  float* dw;                  /* [c_out, c_in * n_ref] */
+} fovi_knnconv_dw_few_args;
+
+int64_t fovi_knnconv_dw_few_workspace_bytes(int64_t batch, int64_t c_in, int64_t c_out, int64_t n_in, int64_t n_out,
+                                            int64_t n_ref, int32_t x_dtype);
+int fovi_knnconv_dw_few(const fovi_knnconv_dw_few_args* args, void* stream);
 
 #ifdef __cplusplus
 }

@@ -1,0 +1,85 @@
+"""``fovi_knnconv_dw_few``: the weight gradient of layers with at most 8 input channels from a bf16
+output gradient, against float64 over the same operands. The products are exact in fp32 (fp32 x
+enters as three bf16 parts that add up to it), so the error is that of fp32 sums: below 1e-5 of
+the result's norm for the few thousand terms here."""
+import pytest
+import torch
+
+from fovi_amd import _lib
+from fovi_amd.arch.knn import KNNConvLayer
+from fovi_amd.sensing.coords import SamplingCoords
+from tests.helpers import assert_close_rel
+from tests.test_dw_tiles import _dw64
+
+
+def _layer(res_in, res_out, k, c_in, c_out, side, device="cuda"):
+    return KNNConvLayer(c_in, c_out, k, SamplingCoords(16, 0.5, res_in, style="isotropic"),
+                        SamplingCoords(16, 0.5, res_out, style="isotropic"), device=device, ref_frame_side_length=side)
+
+
+_SHAPES = [
+    (12, 6, 25, 3, 96, 10, 16),      # V = 100, pad ring, one tile of 96 rows
+    (10, 8, 9, 1, 33, None, 5),      # one channel (32 slots per block, V = 9), images padded to 16
+    (8, 8, 30, 4, 128, 3, 33),       # several neighbours per slot, two tiles of 64 rows
+    (8, 5, 16, 5, 8, 7, 17),         # 30 of 32 columns used
+    (6, 3, 4, 8, 200, None, 1),      # one image, three row tiles
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("res_in,res_out,k,c_in,c_out,side,batch", _SHAPES)
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("layout", ["planes", "rows"])
+def test_dw_few_against_float64(res_in, res_out, k, c_in, c_out, side, batch, dt, layout):
+    layer = _layer(res_in, res_out, k, c_in, c_out, side)
+    g = torch.Generator().manual_seed(c_in)
+    x = torch.randn(batch, c_in, layer.in_coords.shape[0], generator=g).to(dt)
+    dy = torch.randn(batch, c_out, layer.out_coords.shape[0], generator=g).bfloat16()
+    rows = lambda t: t.transpose(1, 2).contiguous().transpose(1, 2) if layout == "rows" else t
+    got = layer._dw_few(rows(x.cuda()), rows(dy.cuda()))
+    assert_close_rel(got.double().cpu(), _dw64(layer, x, dy), 1e-5, f"{dt} {layout}")
+
+
+@pytest.mark.gpu
+def test_dw_few_is_as_exact_as_the_fp32_path():
+    """fp32 x over six orders of magnitude: no further from float64 than the slot sums and the fp32
+    GEMM it replaces (both rounded sums of the same products; twice for the difference of their
+    orders)."""
+    layer = _layer(16, 8, 49, 3, 64, 14)
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(64, 3, layer.in_coords.shape[0], generator=g)
+    x = x * torch.pow(10.0, 6 * torch.rand(x.shape, generator=g) - 3)
+    dy = torch.randn(64, 64, layer.out_coords.shape[0], generator=g).bfloat16()
+    ref = _dw64(layer, x, dy)
+    got = layer._dw_few(x.cuda(), dy.cuda())
+    layer.dw_fused = False
+    _, old = layer._backward(x.cuda(), layer.weight, dy.cuda(), False, True)
+    e = [float((t.double().cpu() - ref).norm() / ref.norm()) for t in (got, old)]
+    assert e[0] <= 2 * e[1] and e[0] < 1e-6, e
+
+
+@pytest.mark.gpu
+def test_autocast_training_step_takes_it_and_non_finite_gradients_show():
+    layer = _layer(12, 6, 25, 3, 64, 10)
+    x = torch.randn(9, 3, layer.in_coords.shape[0], generator=torch.Generator().manual_seed(6)).cuda()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = layer(x)
+    assert y.dtype == torch.bfloat16
+    dy = torch.randn(y.shape, generator=torch.Generator().manual_seed(7)).bfloat16().cuda()
+    y.backward(dy)
+    assert torch.equal(layer.weight.grad, layer._dw_few(x, dy))
+    dy[2, 5, 3] = float("inf")
+    bad = layer._dw_few(x, dy)
+    layer.dw_fused = False
+    _, want = layer._backward(x, layer.weight, dy, False, True)
+    # inf times the zeros of the slots that point 3 does not use, as in the dense product
+    assert torch.equal(torch.isfinite(bad), torch.isfinite(want))
+
+
+def test_dw_few_sizes():
+    lib = _lib.load()
+    assert lib.fovi_knnconv_dw_few_workspace_bytes(128, 3, 96, 4085, 964, 484, _lib.F32) > 0
+    for args in ((0, 3, 96, 4, 4, 9, 0), (8, 9, 96, 4, 4, 9, 0), (8, 3, 96, 4, 4, 9, 2), (8, 3, 0, 4, 4, 9, 0)):
+        assert lib.fovi_knnconv_dw_few_workspace_bytes(*args) == -1
+    assert lib.fovi_knnconv_dw_few(_lib.KnnConvDwFewArgs(), None) != 0
+    assert b"null pointer" in lib.fovi_last_error()
