@@ -3,19 +3,21 @@
 // dy[b, n, o] * x[b, i, c], x fp32 or bf16.
 //
 // The images are the reduction index of the matrix instructions. A first pass lays both operands
-// out with the images adjacent (dyT[n][o][b], xT[i][c][b], bf16, images padded with zeros to
-// 16), so that a lane loads its 8 images of one row or column with one 16-byte load and nothing
-// passes through LDS. fp32 x is split into three bf16 parts by truncation (8 + 8 + 8 significant
+// out in steps of 16 images (dyT[step][n][o][16], xT[step][i][c][16], bf16, padded with zero images),
+// so that a lane loads its 8 images of one row or column with one 16-byte load, the rows of a point
+// adjacent, and nothing passes through LDS (with all images of a row adjacent, [n][o][b], every
+// lane pair read another line: 278 us for the products below). fp32 x is split into three bf16 parts by truncation (8 + 8 + 8 significant
 // bits: exact), each multiplied with dy: the products are exact, the sums fp32, as in an fp32
 // product.
-// A wave owns all rows o of a tile of up to 96 and two blocks of 32 columns, 32 / c_in slots x
-// c_in channels each; for every point of its range it reads the slots' neighbour lists, one
-// neighbour of every slot per round (a slot without one reads a zero row), and skips a block none
+// A wave owns all rows o of a tile of up to 96 and a block of 32 columns, 32 / c_in slots x c_in
+// channels; for every point of its range it reads the slots' neighbour lists, one neighbour of every slot per round (a slot without one reads a zero row), and skips a block none
 // of whose slots has a neighbour (not with a non-finite dy: its product with an empty slot's zero
 // is NaN). Partial tiles per point range go to a workspace and are
 // added in range order.
 // 128 images, 3 -> 96 channels, 4085 -> 964 points, k = 121 in V = 484 slots, x fp32: the slot-sum
-// matrix (717 MB) and an fp32 GEMM over it took 650 + 643 us.
+// matrix (717 MB) and an fp32 GEMM over it took 650 + 643 us; here 151 us, 32 us for the layouts and
+// 20 us for the reduction. Bound by the latency of the operand loads (two column blocks per wave, two
+// waves per SIMD and no load ahead: 227 us).
 #include <type_traits>
 
 #include "common.h"
@@ -25,18 +27,17 @@ namespace {
 
 typedef uint32_t u32x4f __attribute__((ext_vector_type(4)));
 
-constexpr int DF_CT = 2;                 // column blocks per wave
 constexpr int DF_WAVES = 4;
 
 // ---- operands with the images adjacent ------------------------------------------------------
-// out[(fast * of + slow * os) * bp + b], planes of `plane` elements apart for the parts; a block
-// takes 64 fast indices of one slow index and 64 images through LDS: reads run along the fast
-// dimension of the input, writes along the images.
+// out[((b / 16) * rows + fast * of + slow * os) * 16 + b % 16], `plane` elements apart for the parts;
+// a block takes 64 fast indices of one slow index and 64 images through LDS: reads run along the
+// fast dimension of the input, a thread writes 8 images of a row.
 struct LayoutParams {
   const void* in;
   int64_t B, F, S, sb, sf, ss;           // images, fast and slow counts, their element strides
   uint16_t* out;
-  int64_t of, os, bp, plane;
+  int64_t of, os, rows, bp, plane;
   int32_t* flag;                         // set if a value is not finite (or NULL)
 };
 
@@ -53,16 +54,20 @@ __global__ __launch_bounds__(256) void images_adjacent_kernel(LayoutParams p, ui
     tile[k][threadIdx.x & 63] = f < p.F && b < p.B ? in[b * p.sb + f * p.sf] : T(0);
   }
   __syncthreads();
-  // 32 pairs of images x 8 fast indices per pass: 4-byte stores
-  for (int k = threadIdx.x >> 5; k < 64; k += 8) {
-    const int64_t f = f0 + k, b = b0 + 2 * (threadIdx.x & 31);
+  for (int k = threadIdx.x; k < 512; k += 256) {
+    const int64_t f = f0 + (k & 63), b = b0 + 8 * (k >> 6);
     if (f >= p.F || b >= p.bp) continue;
-    uint16_t part[2][NS];
+    uint32_t part[NS][4];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const T v = tile[2 * (threadIdx.x & 31) + u][k];
+    for (int q = 0; q < NS; ++q)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) part[q][u] = 0u;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const T v = tile[8 * (k >> 6) + u][k & 63];
+      const int sh = (u & 1) * 16;
       if constexpr (NS == 1) {
-        part[u][0] = v;
+        part[0][u >> 1] |= static_cast<uint32_t>(v) << sh;
         if (p.flag && (v & 0x7f80u) == 0x7f80u) *p.flag = 1;
       } else {
         // by truncation: the parts add up to v exactly; a non-finite v is its own first part
@@ -71,145 +76,123 @@ __global__ __launch_bounds__(256) void images_adjacent_kernel(LayoutParams p, ui
         const bool fin = (bits & 0x7f800000u) != 0x7f800000u;
         const float r1 = fin ? v - h : 0.0f;
         const float m = __uint_as_float(__float_as_uint(r1) & 0xffff0000u);
-        part[u][0] = static_cast<uint16_t>(bits >> 16);
-        if (!fin && (bits & 0x007fffffu) && !(bits & 0x007f0000u)) part[u][0] |= 1;   // NaN stays NaN
-        part[u][1] = static_cast<uint16_t>(__float_as_uint(m) >> 16);
-        part[u][NS - 1] = static_cast<uint16_t>(__float_as_uint(r1 - m) >> 16);
+        uint32_t hi = bits >> 16;
+        if (!fin && (bits & 0x007fffffu) && !(bits & 0x007f0000u)) hi |= 1u;   // NaN stays NaN
+        part[0][u >> 1] |= hi << sh;
+        part[1][u >> 1] |= (__float_as_uint(m) >> 16) << sh;
+        part[NS - 1][u >> 1] |= (__float_as_uint(r1 - m) >> 16) << sh;
       }
     }
-    uint16_t* o = p.out + (f * p.of + s * p.os) * p.bp + b;
+    uint16_t* o = p.out + ((b >> 4) * p.rows + f * p.of + s * p.os) * 16 + (b & 8);
 #pragma unroll
     for (int q = 0; q < NS; ++q)
-      *reinterpret_cast<uint32_t*>(o + q * p.plane) = part[0][q] | static_cast<uint32_t>(part[1][q]) << 16;
+      *reinterpret_cast<u32x4f*>(o + q * p.plane) = u32x4f{part[q][0], part[q][1], part[q][2], part[q][3]};
   }
 }
 
-__global__ __launch_bounds__(256) void zero_rows_kernel(uint16_t* out, int64_t count, int64_t plane, int ns,
+// the zero row (c_in x 16 values) of every step and part, and the flag
+__global__ __launch_bounds__(128) void zero_rows_kernel(uint16_t* out, int count, int64_t step, int64_t plane, int ns,
                                                         int32_t* flag) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i == 0) *flag = 0;
-  if (i < count)
-    for (int q = 0; q < ns; ++q) out[q * plane + i] = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
+  if (static_cast<int>(threadIdx.x) < count)
+    for (int q = 0; q < ns; ++q) out[q * plane + blockIdx.x * step + threadIdx.x] = 0;
 }
 
 // ---- the products ------------------------------------------------------------------------------
 struct DwFewParams {
-  const uint16_t* dyt;                   // [n_out][c_out][bp]
-  const uint16_t* xt;                    // [parts][n_in + 1][c_in][bp], row n_in zero
+  const uint16_t* dyt;                   // [bp / 16][n_out][c_out][16]
+  const uint16_t* xt;                    // [parts][bp / 16][n_in + 1][c_in][16], row n_in zero
   int64_t plane;
   int C, Cout, Nin, Nout, V, K, bp;
   int slots;                             // slots per column block: 32 / c_in
-  int n_ct, per;                         // column tiles (of DF_CT blocks), points per range
+  int n_ct, per;                         // column blocks, points per range
   const int32_t* slot_ptr;
   const int32_t* nbr;
   const int32_t* flag;                   // dy holds a non-finite value
-  float* part;                           // [ranges][o tiles][n_ct][MB * 32][DF_CT * 32]
+  float* part;                           // [ranges][o tiles][n_ct][MB * 32][32]
 };
 
 template <int MB, int NS>
-__global__ __launch_bounds__(DF_WAVES * 64, 2) void knnconv_dw_few_kernel(DwFewParams p, int ct_groups) {
+__global__ __launch_bounds__(DF_WAVES * 64, 3) void knnconv_dw_few_kernel(DwFewParams p, int ct_groups, int ranges) {
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ct = static_cast<int>(blockIdx.x % ct_groups) * DF_WAVES + wave;
-  const int range = blockIdx.x / ct_groups;
+  const int lb = static_cast<int>(xcd_tile(blockIdx.x, gridDim.x));   // a range's column tiles share an L2
+  const int ct = lb % ct_groups * DF_WAVES + wave;
+  const int range = lb / ct_groups;
+  if (range >= ranges) return;
   const int o0 = blockIdx.y * MB * 32;
   if (ct >= p.n_ct) return;              // no barrier follows
   const int n0 = range * p.per, n1 = min(p.Nout, n0 + p.per);
 
-  // this lane's column of each block: slot v[b], channel c (columns past the slots: none)
-  int v[DF_CT];
-  const int c = l32 % p.C;
-#pragma unroll
-  for (int b = 0; b < DF_CT; ++b) {
-    const int s = l32 / p.C;
-    v[b] = s < p.slots ? (ct * DF_CT + b) * p.slots + s : p.V;
-    if (v[b] >= p.V) v[b] = -1;
-  }
+  // this lane's column: slot v, channel c (columns past the slots: none)
+  const int c = l32 % p.C, sl = l32 / p.C;
+  int v = sl < p.slots ? ct * p.slots + sl : p.V;
+  if (v >= p.V) v = -1;
   uint32_t oa[MB];                       // row offsets of dyT within a point
 #pragma unroll
   for (int m = 0; m < MB; ++m) {
     const int o = min(o0 + m * 32 + l32, p.Cout - 1);
-    oa[m] = static_cast<uint32_t>(o) * p.bp + 8 * h;
+    oa[m] = static_cast<uint32_t>(o) * 16 + 8 * h;
   }
 
-  f32x16 acc[MB][DF_CT];
+  f32x16 acc[MB];
 #pragma unroll
   for (int m = 0; m < MB; ++m)
 #pragma unroll
-    for (int b = 0; b < DF_CT; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[m][b][r] = 0.0f;
+    for (int r = 0; r < 16; ++r) acc[m][r] = 0.0f;
 
-  auto words = [&](int n, int (&w)[DF_CT]) {
-#pragma unroll
-    for (int b = 0; b < DF_CT; ++b) w[b] = n < n1 && v[b] >= 0 ? p.slot_ptr[static_cast<int64_t>(n) * p.V + v[b]] : 0;
-  };
+  auto word = [&](int n) { return n < n1 && v >= 0 ? p.slot_ptr[static_cast<int64_t>(n) * p.V + v] : 0; };
   auto row = [&](int n, int w, int r) {  // the slot's r-th neighbour, or the zero row
     return r < (w & 0xffff) ? p.nbr[static_cast<int64_t>(n) * p.K + (w >> 16) + r] : p.Nin;
   };
   const bool every = *p.flag != 0;
-  int w[DF_CT], wn[DF_CT], i0[DF_CT];
-  words(n0, w);
-#pragma unroll
-  for (int b = 0; b < DF_CT; ++b) i0[b] = n0 < n1 ? row(n0, w[b], 0) : p.Nin;
-  words(n0 + 1, wn);
+  const int64_t dstep = static_cast<int64_t>(p.Nout) * p.Cout * 16, xstep = static_cast<int64_t>(p.Nin + 1) * p.C * 16;
+  const int steps = p.bp / 16;
+  struct Ops { bf16x8 a[MB], x[NS]; };
+  int w = word(n0), i0 = n0 < n1 ? row(n0, w, 0) : p.Nin, wn = word(n0 + 1);
   for (int n = n0; n < n1; ++n) {
-    int inx[DF_CT], wnn[DF_CT];          // the next point's first neighbours, the one after's words
+    // the next point's first neighbours, the one after's words
+    const int inx = n + 1 < n1 ? row(n + 1, wn, 0) : p.Nin, wnn = word(n + 2);
+    const uint16_t* dn = p.dyt + static_cast<int64_t>(n) * p.Cout * 16;
+    for (int r = 0; __builtin_amdgcn_ballot_w64((w & 0xffff) > r) != 0 || (every && r == 0); ++r) {
+      const int i = r == 0 ? i0 : row(n, w, r);
+      const uint16_t* xr = p.xt + (static_cast<int64_t>(i) * p.C + c) * 16 + 8 * h;
+      auto fetch = [&](Ops& t, int s) {
 #pragma unroll
-    for (int b = 0; b < DF_CT; ++b) inx[b] = n + 1 < n1 ? row(n + 1, wn[b], 0) : p.Nin;
-    words(n + 2, wnn);
-    const uint16_t* dn = p.dyt + static_cast<int64_t>(n) * p.Cout * p.bp;
-    for (int r = 0;; ++r) {
-      bool on[DF_CT];
-      const uint16_t* xb[DF_CT];
-      bool any = false;
+        for (int m = 0; m < MB; ++m) t.a[m] = *reinterpret_cast<const bf16x8*>(dn + s * dstep + oa[m]);
 #pragma unroll
-      for (int b = 0; b < DF_CT; ++b) {
-        on[b] = __builtin_amdgcn_ballot_w64((w[b] & 0xffff) > r) != 0 || (every && r == 0);
-        any |= on[b];
-        const int i = r == 0 ? i0[b] : row(n, w[b], r);
-        xb[b] = p.xt + (static_cast<int64_t>(i) * p.C + c) * p.bp + 8 * h;
-      }
-      if (!any) break;
-      // the blocks of this round (uniform): one loop each, so that no product is conditional
-      auto run = [&](auto first, auto last) __attribute__((always_inline)) {
-        constexpr int B0 = decltype(first)::value, B1 = decltype(last)::value;
-#pragma unroll 1
-        for (int k = 0; k < p.bp; k += 16) {
-          bf16x8 a[MB], x[B1 - B0][NS];
-#pragma unroll
-          for (int m = 0; m < MB; ++m) a[m] = *reinterpret_cast<const bf16x8*>(dn + oa[m] + k);
-#pragma unroll
-          for (int b = B0; b < B1; ++b)
-#pragma unroll
-            for (int q = 0; q < NS; ++q) x[b - B0][q] = *reinterpret_cast<const bf16x8*>(xb[b] + q * p.plane + k);
-#pragma unroll
-          for (int b = B0; b < B1; ++b)
-#pragma unroll
-            for (int q = NS - 1; q >= 0; --q)          // small parts first
-#pragma unroll
-              for (int m = 0; m < MB; ++m)
-                acc[m][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[m], x[b - B0][q], acc[m][b], 0, 0, 0);
-        }
+        for (int q = 0; q < NS; ++q) t.x[q] = *reinterpret_cast<const bf16x8*>(xr + s * xstep + q * p.plane);
       };
-      typedef std::integral_constant<int, 0> I0;
-      typedef std::integral_constant<int, 1> I1;
-      typedef std::integral_constant<int, 2> I2;
-      if (on[0] && on[1]) run(I0(), I2());
-      else if (on[0]) run(I0(), I1());
-      else run(I1(), I2());
-    }
+      auto multiply = [&](const Ops& t) {
 #pragma unroll
-    for (int b = 0; b < DF_CT; ++b) { w[b] = wn[b]; wn[b] = wnn[b]; i0[b] = inx[b]; }
+        for (int q = NS - 1; q >= 0; --q)          // small parts first
+#pragma unroll
+          for (int m = 0; m < MB; ++m) acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.a[m], t.x[q], acc[m], 0, 0, 0);
+      };
+      // the next 16 images' operands are loaded while these are multiplied (the last step loads
+      // its own again: a conditional load would make every wait a full one)
+      Ops t0, t1;
+      fetch(t0, 0);
+      for (int s = 0;;) {
+        int nx = min(s + 1, steps - 1);
+        fetch(t1, nx);
+        multiply(t0);
+        if (nx == s) break;
+        s = nx;
+        nx = min(s + 1, steps - 1);
+        fetch(t0, nx);
+        multiply(t1);
+        if (nx == s) break;
+        s = nx;
+      }
+    }
+    w = wn; wn = wnn; i0 = inx;
   }
-  float* out = p.part + ((static_cast<int64_t>(range) * gridDim.y + blockIdx.y) * p.n_ct + ct) * (MB * 32 * DF_CT * 32);
+  float* out = p.part + ((static_cast<int64_t>(range) * gridDim.y + blockIdx.y) * p.n_ct + ct) * (MB * 32 * 32);
 #pragma unroll
   for (int m = 0; m < MB; ++m)
 #pragma unroll
-    for (int b = 0; b < DF_CT; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        out[(m * 32 + 8 * (r >> 2) + 4 * h + (r & 3)) * (DF_CT * 32) + b * 32 + l32] = acc[m][b][r];
+    for (int r = 0; r < 16; ++r) out[(m * 32 + 8 * (r >> 2) + 4 * h + (r & 3)) * 32 + l32] = acc[m][r];
 }
 
 __global__ __launch_bounds__(256) void knnconv_dw_few_reduce_kernel(DwFewParams p, int mb, int ranges, int o_tiles,
@@ -220,9 +203,8 @@ __global__ __launch_bounds__(256) void knnconv_dw_few_reduce_kernel(DwFewParams 
   const int c = static_cast<int>((t / p.V) % p.C), o = static_cast<int>(t / (static_cast<int64_t>(p.V) * p.C));
   const int blk = v / p.slots, col = (v % p.slots) * p.C + c;
   const int rows = mb * 32;
-  const float* src = p.part + (static_cast<int64_t>(o / rows) * p.n_ct + blk / DF_CT) * (rows * DF_CT * 32) +
-                     (o % rows) * (DF_CT * 32) + (blk % DF_CT) * 32 + col;
-  const int64_t stride = static_cast<int64_t>(o_tiles) * p.n_ct * rows * DF_CT * 32;
+  const float* src = p.part + (static_cast<int64_t>(o / rows) * p.n_ct + blk) * (rows * 32) + (o % rows) * 32 + col;
+  const int64_t stride = static_cast<int64_t>(o_tiles) * p.n_ct * rows * 32;
   float sum = 0.0f;
   int s = 0;
   for (; s + 8 <= ranges; s += 8) {
@@ -246,34 +228,34 @@ bool few_plan(int64_t B, int64_t C, int64_t Cout, int64_t Nin, int64_t Nout, int
     return false;
   constexpr int64_t lim = int64_t(1) << 31;
   f.bp = (B + 15) / 16 * 16;
-  if (f.bp >= (1 << 20) || Cout >= (1 << 20) || Nin >= lim - 1 || Nout >= lim || V >= (1 << 20) || Cout * f.bp >= lim)
+  if (f.bp >= (1 << 20) || Cout >= (1 << 20) || Nin >= lim - 1 || Nout >= lim || V >= (1 << 20) || Cout * f.bp >= lim || Cout * 16 >= lim)
     return false;
   f.parts = x_dtype == FOVI_F32 ? 3 : 1;
   f.slots = static_cast<int>(32 / C);
-  const int64_t blocks = (V + f.slots - 1) / f.slots;
-  f.n_ct = static_cast<int>((blocks + DF_CT - 1) / DF_CT);
-  // tiles of up to 96 rows (128 rows x 2 blocks spill their accumulators), as even as they come
+  f.n_ct = static_cast<int>((V + f.slots - 1) / f.slots);
+  // tiles of up to 96 rows (accumulators and two steps' operands for three waves per SIMD), as even
+  // as they come
   const int64_t row_blocks = (Cout + 31) / 32;
   f.o_tiles = static_cast<int>((row_blocks + 2) / 3);
   f.mb = static_cast<int>((row_blocks + f.o_tiles - 1) / f.o_tiles);
   // point ranges: about 3072 waves in all (three per SIMD), each range at least one point
   const int64_t tiles = static_cast<int64_t>(f.n_ct) * f.o_tiles;
-  int64_t ranges = (3072 + tiles - 1) / tiles;
+  int64_t ranges = 3072 / tiles > 0 ? 3072 / tiles : 1;
   if (ranges > Nout) ranges = Nout;
   const int64_t per = (Nout + ranges - 1) / ranges;
   f.per = static_cast<int>(per);
   f.ranges = static_cast<int>((Nout + per - 1) / per);
   f.dyt = (Nout * Cout * f.bp + 63) / 64 * 64;
   f.xt = ((Nin + 1) * C * f.bp + 63) / 64 * 64;
-  f.part = static_cast<int64_t>(f.ranges) * tiles * f.mb * 32 * DF_CT * 32;
+  f.part = static_cast<int64_t>(f.ranges) * tiles * f.mb * 32 * 32;
   return true;
 }
 
 template <typename InT, int NS>
-int lay_out(const void* in, int64_t B, int64_t C, int64_t N, const int64_t* st, uint16_t* out, int64_t bp, int64_t plane,
-            int32_t* flag, hipStream_t s) {
+int lay_out(const void* in, int64_t B, int64_t C, int64_t N, const int64_t* st, uint16_t* out, int64_t out_rows,
+            int64_t bp, int64_t plane, int32_t* flag, hipStream_t s) {
   LayoutParams p;
-  p.in = in; p.B = B; p.sb = st[0]; p.out = out; p.bp = bp; p.plane = plane; p.flag = flag;
+  p.in = in; p.B = B; p.sb = st[0]; p.out = out; p.bp = bp; p.plane = plane; p.rows = out_rows; p.flag = flag;
   const bool rows = st[1] == 1 && C > 1;         // channels adjacent: they are the fast dimension
   p.F = rows ? C : N; p.S = rows ? N : C;
   p.sf = rows ? st[1] : st[2]; p.ss = rows ? st[2] : st[1];
@@ -288,8 +270,8 @@ int lay_out(const void* in, int64_t B, int64_t C, int64_t N, const int64_t* st, 
 template <int NS>
 int launch_few(const DwFewParams& p, const FewPlan& f, hipStream_t s) {
   const int groups = (f.n_ct + DF_WAVES - 1) / DF_WAVES;
-  const dim3 grid(static_cast<unsigned>(static_cast<int64_t>(groups) * f.ranges), static_cast<unsigned>(f.o_tiles));
-  const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(DF_WAVES * 64), 0, s, p, groups); };
+  const dim3 grid(static_cast<unsigned>((static_cast<int64_t>(groups) * f.ranges + 7) / 8 * 8), static_cast<unsigned>(f.o_tiles));
+  const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(DF_WAVES * 64), 0, s, p, groups, f.ranges); };
   if (f.mb == 1) go(knnconv_dw_few_kernel<1, NS>);
   else if (f.mb == 2) go(knnconv_dw_few_kernel<2, NS>);
   else go(knnconv_dw_few_kernel<3, NS>);
@@ -330,13 +312,13 @@ extern "C" int fovi_knnconv_dw_few(const fovi_knnconv_dw_few_args* a, void* stre
   uint16_t* dyt = reinterpret_cast<uint16_t*>(part + f.part);
   uint16_t* xt = dyt + f.dyt;
   int32_t* flag = reinterpret_cast<int32_t*>(xt + f.parts * f.xt);
-  const int64_t zero = a->c_in * f.bp;
-  hipLaunchKernelGGL(zero_rows_kernel, dim3(static_cast<unsigned>((zero + 255) / 256)), dim3(256), 0, s,
-                     xt + a->n_in * zero, zero, f.xt, f.parts, flag);
+  const int64_t x_rows = (a->n_in + 1) * a->c_in;
+  hipLaunchKernelGGL(zero_rows_kernel, dim3(static_cast<unsigned>(f.bp / 16)), dim3(128), 0, s,
+                     xt + a->n_in * a->c_in * 16, static_cast<int>(a->c_in) * 16, x_rows * 16, f.xt, f.parts, flag);
   if (check_launch("fovi_knnconv_dw_few(zero row)")) return 1;
-  if (lay_out<uint16_t, 1>(a->dy, a->batch, a->c_out, a->n_out, a->dy_stride, dyt, f.bp, 0, flag, s)) return 1;
-  if (a->x_dtype == FOVI_F32 ? lay_out<float, 3>(a->x, a->batch, a->c_in, a->n_in, a->x_stride, xt, f.bp, f.xt, nullptr, s)
-                             : lay_out<uint16_t, 1>(a->x, a->batch, a->c_in, a->n_in, a->x_stride, xt, f.bp, f.xt,
+  if (lay_out<uint16_t, 1>(a->dy, a->batch, a->c_out, a->n_out, a->dy_stride, dyt, a->n_out * a->c_out, f.bp, 0, flag, s)) return 1;
+  if (a->x_dtype == FOVI_F32 ? lay_out<float, 3>(a->x, a->batch, a->c_in, a->n_in, a->x_stride, xt, x_rows, f.bp, f.xt, nullptr, s)
+                             : lay_out<uint16_t, 1>(a->x, a->batch, a->c_in, a->n_in, a->x_stride, xt, x_rows, f.bp, f.xt,
                                                     nullptr, s))
     return 1;
   p.dyt = dyt; p.xt = xt; p.plane = f.xt;
