@@ -80,7 +80,7 @@ class RetinalTransform(nn.Module):
     @torch.autocast(device_type="cuda", enabled=False)
     def forward(self, x, fix_loc, fixation_size=None, **kwargs):
         fixation_size = self._check_fixation_size(fixation_size, x.shape[0])
-        fix_loc = self._check_fix_loc(fix_loc, x.shape[0])
+        fix_loc = self._check_fix_loc(fix_loc, x.shape[0], device="cpu")     # the sampler sends it on
         if self.pre_transforms is not None and self.training:
             x = self.pre_transforms(x.clone())
         x = self.sampler(x, fix_loc=fix_loc, fixation_size=fixation_size, **kwargs)
@@ -100,7 +100,7 @@ class RetinalTransform(nn.Module):
         bsz, n_fix = x.shape[0], fix_loc.shape[1]
         if tuple(fix_loc.shape) != (bsz, n_fix, 2):
             raise ValueError(f"fix_loc must be [{bsz}, F, 2]; got {tuple(fix_loc.shape)}")
-        loc = torch.as_tensor(fix_loc).to(dtype=self.dtype, device=self.device).reshape(bsz * n_fix, 2)
+        loc = torch.as_tensor(fix_loc).to(dtype=self.dtype).reshape(bsz * n_fix, 2)
         size = torch.as_tensor(fixation_size).detach().cpu()
         if tuple(size.shape) != (bsz, n_fix, 2):
             raise ValueError(f"fixation_size must be [{bsz}, {n_fix}, 2]; got {tuple(size.shape)}")
@@ -150,8 +150,9 @@ class RetinalTransform(nn.Module):
             assert fixation_size.shape[0] == batch_size
         return fixation_size
 
-    def _check_fix_loc(self, fix_loc, batch_size):
-        """fp32 ``[B, 2]`` (h, w) fixation centres (reference ``retina.py:211-237``)."""
+    def _check_fix_loc(self, fix_loc, batch_size, device=None):
+        """fp32 ``[B, 2]`` (h, w) fixation centres (reference ``retina.py:211-237``), on the
+        transform's device or ``device``."""
         if fix_loc is None:
             fix_loc = np.array([0.5, 0.5])
         elif isinstance(fix_loc, (float, int)):
@@ -164,4 +165,4 @@ class RetinalTransform(nn.Module):
             fix_loc = np.expand_dims(np.array(fix_loc.squeeze()), axis=0).repeat(batch_size, axis=0)
         else:
             assert fix_loc.shape[0] == batch_size
-        return torch.tensor(fix_loc, dtype=self.dtype, device=self.device)
+        return torch.tensor(fix_loc, dtype=self.dtype, device=self.device if device is None else device)

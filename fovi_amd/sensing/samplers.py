@@ -35,7 +35,16 @@ def fixation_half_sizes(fixation_size, n):
     """
     fs = fixation_size
     if isinstance(fs, (tuple, list, np.ndarray)):
-        fs = torch.tensor(np.asarray(fs))
+        fs = np.asarray(fs)
+        if fs.ndim == 2 and fs.shape == (n, 2) and fs.dtype in (np.int64, np.int32, np.float32, np.float64):
+            # the usual calls in numpy: a handful of tensor operations cost a small launch's time
+            wide = fs.dtype == np.float64
+            half = (fs if wide else fs.astype(np.float32)) / fs.dtype.type(2) if fs.dtype.kind == "f" \
+                else fs.astype(np.float32) / np.float32(2)
+            if not np.isfinite(half).all():
+                raise ValueError("fixation_size must be finite")
+            return torch.from_numpy(np.ascontiguousarray(half, dtype=np.float64)), int(wide)
+        fs = torch.tensor(fs)
     fs = torch.as_tensor(fs).detach().cpu()
     if fs.ndim == 1:
         fs = fs.unsqueeze(0)
@@ -104,26 +113,41 @@ class GridSampler(BaseGridSampler):
 
         ``fix_loc [V, 2]`` (h, w) in [0, 1]; ``fixation_size [V, 2]`` (h, w)
         pixels; ``view_image [V]`` image index per view (default: view v
-        reads image v).
+        reads image v). The tables are on the device when this returns (any stream may use them).
         """
-        fix_loc = torch.as_tensor(fix_loc, dtype=torch.float32).reshape(-1, 2)
+        return self._make_views(fix_loc, fixation_size, n_img, device, view_image, blocking=True)
+
+    def _make_views(self, fix_loc, fixation_size, n_img, device, view_image, blocking):
+        """``prepare_views``; with ``blocking`` False the tables are sent on the current stream without
+        waiting for it, for a launch on that stream."""
+        # checked on the host (a device check is five launches and a wait), then sent with the
+        # sizes and the map in one copy from pinned memory
+        fix_loc = torch.as_tensor(fix_loc).detach().to(device="cpu", dtype=torch.float32).reshape(-1, 2)
         # non-finite centres or sizes would put taps at undefined pixel coordinates
-        if not bool(torch.isfinite(fix_loc).all()):
+        if not np.isfinite(fix_loc.numpy()).all():
             raise ValueError("fix_loc must be finite")
-        fix_loc = fix_loc.to(device).contiguous()
         n_views = fix_loc.shape[0]
         half, wide = fixation_half_sizes(fixation_size, n_views)
-        vmap = None
+        vi = None
         if view_image is not None:
             vi = torch.as_tensor(view_image).reshape(-1)
             if vi.numel() != n_views:
                 raise ValueError("view_image must have one entry per view")
             if int(vi.min()) < 0 or int(vi.max()) >= n_img:
                 raise ValueError(f"view_image entries must be in [0, {n_img})")
-            vmap = vi.to(device=device, dtype=torch.int32).contiguous()
         elif n_views > n_img:
             raise ValueError(f"{n_views} views of {n_img} images need a view_image map")
-        return _Views(fix_loc, half.to(device), wide, vmap, n_views, n_img)
+        device = torch.device(device)
+        cuda = device.type == "cuda"
+        host = torch.empty(n_views * 7, dtype=torch.int32, pin_memory=cuda)
+        host[:4 * n_views].view(torch.float64).copy_(half.reshape(-1))
+        host[4 * n_views:6 * n_views].view(torch.float32).copy_(fix_loc.reshape(-1))
+        if vi is not None:
+            host[6 * n_views:].copy_(vi)
+        dev = host.to(device, non_blocking=cuda and not blocking)
+        return _Views(dev[4 * n_views:6 * n_views].view(torch.float32).view(n_views, 2),
+                      dev[:4 * n_views].view(torch.float64).view(n_views, 2), wide,
+                      None if vi is None else dev[6 * n_views:], n_views, n_img)
 
     def sample_views(self, img, fix_loc=None, fixation_size=None, view_image=None, out=None, out_dtype=None,
                      return_grid=False, views=None):
@@ -139,7 +163,7 @@ class GridSampler(BaseGridSampler):
         n_img, ch, hh, ww = img.shape
         dev = img.device
         if views is None:
-            views = self.prepare_views(fix_loc, fixation_size, n_img, dev, view_image)
+            views = self._make_views(fix_loc, fixation_size, n_img, dev, view_image, blocking=False)
         elif views.n_img > n_img:
             raise ValueError(f"views were prepared for {views.n_img} images, got {n_img}")
         n_views = views.n_views
