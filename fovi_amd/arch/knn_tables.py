@@ -1301,18 +1301,18 @@ IMG_SAMPLE = 4            # windows looked at when the group size is chosen
 def spatial_order(coords, leaf=IMG_WINDOW):
     """A permutation (int32) of the points ``coords [N, D]`` in which every run of about ``leaf``
     points is compact: recursive median splits along the widest axis."""
-    pts = torch.as_tensor(coords).detach().cpu().to(torch.float64).numpy()
+    pts = torch.as_tensor(coords).detach().cpu().to(torch.float64).t().contiguous().numpy()
     out = []
-    stack = [np.arange(pts.shape[0])]
+    stack = [np.arange(pts.shape[1])]
     while stack:
         idx = stack.pop()
         if idx.size <= leaf:
-            out.append(idx)
+            out.append(np.sort(idx))
             continue
-        sub = pts[idx]
-        axis = int(np.argmax(sub.max(0) - sub.min(0)))
+        sub = np.take(pts, idx, axis=1)
+        axis = int(np.argmax(sub.max(1) - sub.min(1)))
         half = leaf * (-(-idx.size // leaf) // 2)           # whole leaves on the first side
-        idx = idx[np.argsort(sub[:, axis], kind="stable")]
+        idx = idx[np.argpartition(sub[axis], half)]
         stack += [idx[half:], idx[:half]]
     return torch.from_numpy(np.concatenate(out)).to(torch.int32)
 
