@@ -529,13 +529,13 @@ extern "C" int fovi_knnconv_pack_weight_img(const float* w_ref, int64_t c_out, i
 }
 
 // Host: groups of `pp` output points with similar slot sets. Within each window of `window`
-// consecutive points (of point_order, or of the index order) a group starts at the unassigned point with most slots and takes, one at a
-// time, the point that adds fewest slots to the union (ties: most slots shared, then the lowest
-// index). With ent == NULL only the groups' union sizes are counted, over every `stride`-th window.
+// consecutive points (of point_order, or of the index order) a group starts at the unassigned point
+// with most slots and takes, one at a time, the point that adds fewest slots to the union (ties: most
+// slots shared, then the lowest index). With ent == NULL only the groups' union sizes are counted, over every `stride`-th window.
 extern "C" int64_t fovi_knnconv_img_tables(const int32_t* slot_ptr, const int32_t* nbr, int64_t n_out, int64_t k,
                                            int64_t n_ref, const int32_t* slot_order, const int32_t* point_order,
-                                           int32_t pp, int64_t window, int64_t stride, uint32_t* ent, int32_t* points, int32_t* nact,
-                                           double* mean_union) {
+                                           int32_t pp, int64_t window, int64_t stride, uint32_t* ent,
+                                           int32_t* points, int32_t* nact, double* mean_union) {
   using namespace fovi;
   clear_error();
   if (!slot_ptr || (!nbr && ent) || n_out <= 0 || k <= 0 || k > 32767 || n_ref <= 0 || pp <= 0 || window <= 0 ||
@@ -551,7 +551,14 @@ extern "C" int64_t fovi_knnconv_img_tables(const int32_t* slot_ptr, const int32_
       }
   auto point = [&](int64_t i) -> int64_t { return point_order ? point_order[i] : i; };
   const int64_t words = (n_ref + 63) / 64;
+  // in registers: the host baseline's popcount builtin is a library call
+  auto pop = [](uint64_t b) -> int32_t {
+    b -= (b >> 1) & 0x5555555555555555ull;
+    b = (b & 0x3333333333333333ull) + ((b >> 2) & 0x3333333333333333ull);
+    return static_cast<int32_t>((((b + (b >> 4)) & 0x0f0f0f0f0f0f0f0full) * 0x0101010101010101ull) >> 56);
+  };
   std::vector<uint64_t> bits(static_cast<size_t>(window * words));
+  std::vector<int32_t> used_n(static_cast<size_t>(window));
   std::vector<int64_t> group(static_cast<size_t>(pp)), left;
   std::vector<uint64_t> uni(static_cast<size_t>(words));
   int64_t groups = 0;
@@ -559,9 +566,13 @@ extern "C" int64_t fovi_knnconv_img_tables(const int32_t* slot_ptr, const int32_
   for (int64_t w0 = 0; w0 < n_out; w0 += window * stride) {
     const int64_t wn = n_out - w0 < window ? n_out - w0 : window;
     std::fill(bits.begin(), bits.end(), 0);
-    for (int64_t i = 0; i < wn; ++i)
+    for (int64_t i = 0; i < wn; ++i) {
+      const int32_t* sp = slot_ptr + point(w0 + i) * n_ref;
       for (int64_t v = 0; v < n_ref; ++v)
-        if (slot_ptr[point(w0 + i) * n_ref + v] & 0xffff) bits[i * words + (v >> 6)] |= uint64_t(1) << (v & 63);
+        bits[i * words + (v >> 6)] |= static_cast<uint64_t>((sp[v] & 0xffff) != 0) << (v & 63);
+      used_n[i] = 0;
+      for (int64_t w = 0; w < words; ++w) used_n[i] += pop(bits[i * words + w]);
+    }
     left.clear();
     for (int64_t i = 0; i < wn; ++i) left.push_back(i);
     while (!left.empty()) {
@@ -572,13 +583,12 @@ extern "C" int64_t fovi_knnconv_img_tables(const int32_t* slot_ptr, const int32_
         if (pp > 1) {
           int64_t bs = INT64_MIN;
           for (size_t c = 0; c < left.size(); ++c) {
-            int64_t add = 0, shared = 0;
-            for (int64_t w = 0; w < words; ++w) {
-              const uint64_t b = bits[left[c] * words + w];
-              add += __builtin_popcountll(b & ~uni[w]);
-              shared += __builtin_popcountll(b & uni[w]);
+            int64_t add = used_n[left[c]];
+            if (n > 0) {
+              add = 0;
+              for (int64_t w = 0; w < words; ++w) add += pop(bits[left[c] * words + w] & ~uni[w]);
             }
-            const int64_t score = n == 0 ? add : shared - add * 65536;
+            const int64_t score = n == 0 ? add : used_n[left[c]] - add - add * 65536;   // shared, then added
             if (score > bs) { bs = score; best = c; }
           }
         }
@@ -588,7 +598,7 @@ extern "C" int64_t fovi_knnconv_img_tables(const int32_t* slot_ptr, const int32_
         group[n++] = i;
       }
       int64_t na = 0;
-      for (int64_t w = 0; w < words; ++w) na += __builtin_popcountll(uni[w]);
+      for (int64_t w = 0; w < words; ++w) na += pop(uni[w]);
       sum += static_cast<double>(na);
       if (ent) {
         for (int64_t q = 0; q < pp; ++q) points[groups * pp + q] = q < n ? static_cast<int32_t>(point(w0 + group[q])) : -1;
