@@ -16,16 +16,22 @@ also what the reference returns (``F.linear(...).transpose(1,2)``,
 Compute dtype: bf16 inputs, or any input under ``torch.autocast('cuda',
 dtype=torch.bfloat16)``, run the bf16 MFMA kernel with fp32 accumulation and
 return bf16 (the reference's autocast behaviour); fp32 inputs run the fp32
-kernel. ``Fp8Activations`` inputs (``layer.quantize_input``), or any input
+kernel. From ``IMG_MIN_BATCH`` images on, layers of at least 16 channels run
+the image-row kernel where it has less to do: matrix rows are images of a few
+neighbouring points, and only the slots those points use are visited (the
+same results for finite weights; any input layout, copied to channels-last
+rows). ``Fp8Activations`` inputs (``layer.quantize_input``), or any input
 when ``layer.fp8`` is set, run the e4m3 MFMA kernel (per-tensor activation
 scale, per-output-channel weight scale ``amax|W[o]|/448``, fp32 accumulation,
 bf16 output); the reference has no fp8 path.
 
-Backward (autograd through ``_KnnConvFn``): the slot sums again
-(``fovi_knnconv_slotsum``) for ``dW = dy^T a``, ``dy W`` as a library GEMM and
-its transposed gather (``fovi_knnconv_bwd_x``, over the inverse neighbour
-table, no atomics) for ``dx``; fp32 and bf16 inputs. The fp8 path has no
-backward.
+Backward (autograd through ``_KnnConvFn``; fp32 and bf16 inputs): ``dx`` is the
+forward of the transposed layer (``_TransposedKnnConv``, over the inverse
+neighbour table, no atomics). ``dW`` of bf16 layers runs over each slot's
+(output, input) pairs (``fovi_knnconv_dw``), that of layers of at most 8
+channels with a bf16 output gradient over the images
+(``fovi_knnconv_dw_few``); the others take the slot sums again
+(``fovi_knnconv_slotsum``) and a library GEMM. The fp8 path has no backward.
 """
 from __future__ import annotations
 

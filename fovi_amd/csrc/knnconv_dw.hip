@@ -12,13 +12,13 @@
 // numbered slot-fastest and mapped XCD by XCD, so the V workgroups of a chunk share one L2.
 //
 // Per step of K = 64 pairs (32 with the smaller tiles) the workgroup loads the dy rows and the x
-// rows (16-byte chunks, a full row per 32 or 16 lanes) into LDS in their natural
-// [pair][channel] layout, double buffered one step ahead. Both MFMA operands need the pair index contiguous per lane, which
-// the transposed LDS read ds_read_b64_tr_b16 delivers: within a 16-lane group, lane j
-// addresses four channels of pair row k0 + j/4 and lane i receives channel i of pairs
-// k0 .. k0 + 3. Rows are 576 (320) bytes apart so those reads hit 64 distinct banks.
-// Per-workgroup partial tiles go to a caller workspace; a second kernel sums them into the
-// reference weight layout (column c * V + v), fp32.
+// rows (16-byte chunks, a full row per 32 or 16 lanes) into LDS in their natural [pair][channel]
+// layout, double buffered one step ahead. Both MFMA operands need the pair index contiguous per
+// lane, which the transposed LDS read ds_read_b64_tr_b16 delivers: within a 16-lane group, lane j
+// addresses four channels of pair row k0 + j/4 and lane i receives channel i of pairs k0 ..
+// k0 + 3. Rows are 576 (320) bytes apart so those reads hit 64 distinct banks. Per-workgroup partial
+// tiles go to a caller workspace; a second kernel sums them into the reference weight layout
+// (column c * V + v), fp32.
 #include "common.h"
 
 namespace fovi {

@@ -3,17 +3,17 @@
 // dy[b, n, o] * x[b, i, c], x fp32 or bf16.
 //
 // The images are the reduction index of the matrix instructions. A first pass lays both operands
-// out in steps of 16 images (dyT[step][n][o][16], xT[step][i][c][16], bf16, padded with zero images),
-// so that a lane loads its 8 images of one row or column with one 16-byte load, the rows of a point
-// adjacent, and nothing passes through LDS (with all images of a row adjacent, [n][o][b], every
-// lane pair read another line: 278 us for the products below). fp32 x is split into three bf16 parts by truncation (8 + 8 + 8 significant
-// bits: exact), each multiplied with dy: the products are exact, the sums fp32, as in an fp32
-// product.
+// out in steps of 16 images (dyT[step][n][o][16], xT[step][i][c][16], bf16, padded with zero
+// images), so that a lane loads its 8 images of one row or column with one 16-byte load, the rows of
+// a point adjacent, and nothing passes through LDS (with all images of a row adjacent, [n][o][b],
+// every lane pair read another line: 278 us for the products below). fp32 x is split into three
+// bf16 parts by truncation (8 + 8 + 8 significant bits: exact), each multiplied with dy: the
+// products are exact, the sums fp32, as in an fp32 product.
 // A wave owns all rows o of a tile of up to 96 and a block of 32 columns, 32 / c_in slots x c_in
-// channels; for every point of its range it reads the slots' neighbour lists, one neighbour of every slot per round (a slot without one reads a zero row), and skips a block none
-// of whose slots has a neighbour (not with a non-finite dy: its product with an empty slot's zero
-// is NaN). Partial tiles per point range go to a workspace and are
-// added in range order.
+// channels; for every point of its range it reads the slots' neighbour lists, one neighbour of every
+// slot per round (a slot without one reads a zero row), and skips a block none of whose slots has a
+// neighbour (not with a non-finite dy: its product with an empty slot's zero is NaN). Partial tiles
+// per point range go to a workspace and are added in range order.
 // 128 images, 3 -> 96 channels, 4085 -> 964 points, k = 121 in V = 484 slots, x fp32: the slot-sum
 // matrix (717 MB) and an fp32 GEMM over it took 650 + 643 us; here 151 us, 32 us for the layouts and
 // 20 us for the reduction. Bound by the latency of the operand loads (two column blocks per wave, two
