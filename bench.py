@@ -490,7 +490,7 @@ def main():
                    "batch": 64, "points": 16384, "k": 25, "c_in": 256, "c_out": 256},
         "roofline": {"bound": "mfma", "achieved": round(c3["tflops"], 2), "peak": PEAK_BF16_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(c3["tflops"] / PEAK_BF16_TFLOPS, 4),
-                     "traffic": measured_traffic("knnconv_bf16_v5_kernel")},
+                     "traffic": measured_traffic("knnconv_img_kernel")},
         "cpu_baseline": cpu,
     }
     if "table_s" in c3:
