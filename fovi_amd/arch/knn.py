@@ -695,10 +695,15 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         work, (rb, ib, _) = self._image_plan(bsz)
         if dt != torch.float32 and self._mfma_path(x, dt):
             # the wide-layer kernel visits every slot, one workgroup of 256 points of an image per
-            # CU; a slot costs it 3/4 of the image-row kernel's (C3: 3.2 ms for 25, 2.82 for 16.9)
+            # CU; its time in slots of the image-row kernel, from both sides at V = 9 and 25,
+            # 256 to 16384 points, 8 to 256 images (V = 9, 16384 points, B = 64: bf16 0.78 against
+            # 0.62 ms, e4m3 0.64 against 0.39; V = 25: 3.15 against 2.80 and 2.36 against 1.54; the
+            # same with 24 images in two blocks of 16: 1.20 against 1.32, bf16)
             tiles = bsz * -(-self.out_coords.shape[0] // 256) * -(-self.out_channels // 256)
             pad = -(-self.out_coords.shape[0] // 256) * 256 / self.out_coords.shape[0]
-            if 0.75 * self.ref_coords.shape[0] * pad * (-(-tiles // 256) * 256 / tiles) < work:
+            v = self.ref_coords.shape[0]
+            wide = 0.93 * v + 3.2 if dt == torch.float8_e4m3fn else 0.62 * v + 3.4
+            if wide * pad * (-(-tiles // 256) * 256 / tiles) < work:
                 return False
         hit = self._img.tables.get(rb * 32 // ib)
         return (hit is not None and hit[0] == x.device) or not torch.cuda.is_current_stream_capturing()
