@@ -117,7 +117,9 @@ __global__ __launch_bounds__(IM_THREADS, 2) void knnconv_img_kernel(KnnParams p,
   constexpr int E_BYTES = IM_WAVES * 32 * EW * OES;
   constexpr int S_BYTES = 4 * A_BYTES > E_BYTES ? 4 * A_BYTES : E_BYTES;
   __shared__ __attribute__((aligned(16))) uint8_t smem[S_BYTES];
-  __shared__ int32_t s_pts[8];                     // the group's points (at most 128 / 16)
+  // the group's points (at most 128 / 16): written by the first wave, read by all in the epilogue,
+  // with a barrier between on every path
+  __shared__ int32_t s_pts[8];
 
   const int64_t lb = xcd_tile(blockIdx.x, padded);
   if (lb >= total) return;
@@ -329,6 +331,8 @@ __global__ __launch_bounds__(IM_THREADS, 2) void knnconv_img_kernel(KnnParams p,
       pos1 = cur[1].pos; c1 = cur[1].c;
       barrier();
     }
+  } else {
+    barrier();   // a group none of whose points has a neighbour: s_pts, which every wave reads below
   }
   if (!live) return;
 
