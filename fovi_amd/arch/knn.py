@@ -539,8 +539,10 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
             self._heavy_stride = wide.heavy_stride
             self._hlist_stride = wide.hlist_stride
         self.slot_order = None if order is None else [int(v) for v in order]
-        self._slot_order_dev = None if order is None else torch.tensor(self.slot_order, dtype=torch.int32,
-                                                                          device=dev)
+        # a buffer like the tables beside it: the weight packing kernels read it, so it moves with the layer
+        self.__dict__.pop("_slot_order_dev", None)     # (a plain attribute in layers pickled before)
+        self.register_buffer("_slot_order_dev", None if order is None else
+                             torch.tensor(self.slot_order, dtype=torch.int32, device=dev), persistent=False)
         for dt in (torch.bfloat16, torch.float8_e4m3fn, torch.float32):
             self._packed.pop(("mfma", dt), None)
             self._packed.pop(("image", dt), None)
