@@ -59,6 +59,14 @@ def fixation_half_sizes(fixation_size, n):
     return half.to(torch.float64).contiguous(), int(wide)
 
 
+def _capturing(device):
+    """Whether the current stream of the CUDA ``device`` is being captured."""
+    if device.index in (None, torch.cuda.current_device()):
+        return torch.cuda.is_current_stream_capturing()
+    with torch.cuda.device(device):
+        return torch.cuda.is_current_stream_capturing()
+
+
 class _Views:
     """Device-resident fixation tables of one set of views."""
 
@@ -114,12 +122,19 @@ class GridSampler(BaseGridSampler):
         ``fix_loc [V, 2]`` (h, w) in [0, 1]; ``fixation_size [V, 2]`` (h, w)
         pixels; ``view_image [V]`` image index per view (default: view v
         reads image v). The tables are on the device when this returns (any stream may use them).
+        Not while the stream is being captured: captured calls take views prepared before.
         """
         return self._make_views(fix_loc, fixation_size, n_img, device, view_image, blocking=True)
 
     def _make_views(self, fix_loc, fixation_size, n_img, device, view_image, blocking):
         """``prepare_views``; with ``blocking`` False the tables are sent on the current stream without
         waiting for it, for a launch on that stream."""
+        device = torch.device(device)
+        cuda = device.type == "cuda"
+        if cuda and _capturing(device):
+            # a graph would replay the copy from a host block that is given back after this call
+            raise RuntimeError("fixations cannot be sent to the device while its stream is being captured: "
+                               "call prepare_views before the capture and pass its result as views")
         # checked on the host (a device check is five launches and a wait), then sent with the
         # sizes and the map in one copy from pinned memory
         fix_loc = torch.as_tensor(fix_loc).detach().to(device="cpu", dtype=torch.float32).reshape(-1, 2)
@@ -137,8 +152,6 @@ class GridSampler(BaseGridSampler):
                 raise ValueError(f"view_image entries must be in [0, {n_img})")
         elif n_views > n_img:
             raise ValueError(f"{n_views} views of {n_img} images need a view_image map")
-        device = torch.device(device)
-        cuda = device.type == "cuda"
         host = torch.empty(n_views * 7, dtype=torch.int32, pin_memory=cuda)
         host[:4 * n_views].view(torch.float64).copy_(half.reshape(-1))
         host[4 * n_views:6 * n_views].view(torch.float32).copy_(fix_loc.reshape(-1))
