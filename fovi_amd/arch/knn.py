@@ -58,8 +58,9 @@ __all__ = [
     "register_with_reference",
 ]
 
-# Smallest batch of the image-row kernel.
+# Smallest batch and fewest input channels of the image-row kernel.
 IMG_MIN_BATCH = 8
+IMG_MIN_CHANNELS = 16
 
 _KCHUNK = 64  # reduction chunk of the MFMA kernel; packed weights are padded to it
 
@@ -186,12 +187,22 @@ class _KnnConvFn(torch.autograd.Function):
 
 class _ImageRows:
     """What the image-row kernel keeps per layer: host copies of the CSR tables it builds its own
-    from, the point order, the device tables per group size (at most five), the mean slot unions
-    and the plans per batch size."""
+    from, the point order, the device tables ``(ent, points, nact)`` and the mean slot union per group
+    size, and the plans per batch size."""
 
     def __init__(self, slot_ptr, nbr):
         self.slot_ptr, self.nbr = slot_ptr.cpu(), nbr.cpu()
         self.order, self.tables, self.unions, self.plans = None, {}, {}, {}
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self.tables = {pp: t[-3:] for pp, t in self.tables.items()}    # (the device came first once)
+
+    def groups(self):
+        """Points per group that plans may take: 16 bytes per (point, slot) each, so a layer of more
+        than 8 Mi (point, slot) pairs keeps to one and two (the two that every batch size has a
+        plan for)."""
+        return (1, 2, 4, 8) if self.slot_ptr.numel() <= 8 << 20 else (1, 2)
 
 
 class KNNConvLayer(nn.Module, KNNBaseLayer):
@@ -548,6 +559,17 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
             self._packed.pop(("image", dt), None)
         if self._img is not None:
             self._img.tables = {}
+            if self.in_channels >= IMG_MIN_CHANNELS and 0 < self._k <= 32767 and len(self._img.slot_ptr):
+                for pp in self._img.groups():
+                    self._image_union(pp)
+                    self._image_tables_of(pp, dev)
+
+    def _apply(self, fn, recurse=True):
+        super()._apply(fn, recurse)
+        if self._img is not None:
+            # not buffers: wrappers that broadcast a module's buffers on every step need not send these
+            self._img.tables = {pp: tuple(fn(t) for t in ts) for pp, ts in self._img.tables.items()}
+        return self
 
     def _packed_weight_mfma(self, dtype=torch.bfloat16):
         """Weight in MFMA-fragment order (``fovi_knnconv_pack_weight_mfma``) for the current slot
@@ -626,14 +648,12 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
             eff *= n_ct * 128 * cb / self.out_channels
             for ib in (16, 32, 64, 128):
                 pp = rb * 32 // ib
-                if pp < 1 or (ib > 16 and ib >= 2 * batch):
+                if pp not in img.groups() or (ib > 16 and ib >= 2 * batch):
                     continue
-                if pp not in img.unions:
-                    img.unions[pp] = T.image_row_union(img.slot_ptr, self._point_order(), pp)
                 blocks = -(-batch // ib)
                 groups = -(-n_out // pp) * blocks * n_ct
                 fill = -(-groups // 512) * 512 / groups        # two workgroups on each of 256 CUs
-                work = blocks * ib / batch * img.unions[pp] * eff * fill
+                work = blocks * ib / batch * self._image_union(pp) * eff * fill
                 values = ib * self.in_coords.shape[0] * self.in_channels
                 cost = work * (1.0 + 0.06 * max(0.0, math.log2(values / 2 ** 24)))
                 if best is None or cost < best[0]:
@@ -650,15 +670,24 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
             self._img.order = T.spatial_order(c.cortical if c.cortical is not None else c.cartesian)
         return self._img.order
 
+    def _image_union(self, pp):
+        """Mean number of slots a group of ``pp`` points visits."""
+        img = self._img
+        if pp not in img.unions:
+            img.unions[pp] = T.image_row_union(img.slot_ptr, self._point_order(), pp)
+        return img.unions[pp]
+
     def _image_tables_of(self, pp, device):
-        """The image-row kernel's device tables for groups of ``pp`` points, built once."""
+        """The image-row kernel's tables for groups of ``pp`` points on ``device``: built with the slot
+        order's other tables for every group size a plan may take, so that no call waits for
+        them (16384 points, V = 25: 8 ms for the four sizes, uploads included), and moved with the layer."""
         hit = self._img.tables.get(pp)
-        if hit is None or hit[0] != device:
-            ent, points, nact = T.image_row_tables(self._img.slot_ptr, self._img.nbr, self.slot_order,
-                                                   self._point_order(), pp)
-            hit = (device, ent.to(device), points.to(device), nact.to(device))
+        if hit is None or hit[0].device != device:
+            tables = hit or T.image_row_tables(self._img.slot_ptr, self._img.nbr, self.slot_order,
+                                               self._point_order(), pp)
+            hit = tuple(t.to(device) for t in tables)
             self._img.tables[pp] = hit
-        return hit[1:]
+        return hit
 
     def _packed_weight_image(self, dtype):
         """``(fragments, non-finite flag, w_scale)`` of the image-row kernel's weight
@@ -686,12 +715,13 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
 
     def _image_path(self, x, dt):
         """Whether this call runs the image-row kernel: a batch of at least ``IMG_MIN_BATCH`` (below,
-        most of a block of 16 images would be padding), at least 16 input channels, 32-bit
-        offsets within a block of images, and less estimated work than the wide-layer kernel
-        where that one applies. Under stream capture only with its tables already built (their
-        upload cannot be captured)."""
+        most of a block of 16 images would be padding), at least ``IMG_MIN_CHANNELS`` input channels,
+        32-bit offsets within a block of images, and less estimated work than the wide-layer
+        kernel where that one applies. The choice depends on the layer and the call alone, not on
+        earlier calls (but for a layer unpickled without its tables: their upload cannot be
+        captured)."""
         bsz = x.shape[0]
-        if not (self.image_rows and bsz >= IMG_MIN_BATCH and self.in_channels >= 16 and self._k <= 32767
+        if not (self.image_rows and bsz >= IMG_MIN_BATCH and self.in_channels >= IMG_MIN_CHANNELS and self._k <= 32767
                 and x.shape[2] * (-(-self.in_channels // 16) * 16) * min(bsz, 128) * dt.itemsize < 2 ** 31 - 4096):
             return False
         work, (rb, ib, _) = self._image_plan(bsz)
@@ -708,7 +738,7 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
             if wide * pad * (-(-tiles // 256) * 256 / tiles) < work:
                 return False
         hit = self._img.tables.get(rb * 32 // ib)
-        return (hit is not None and hit[0] == x.device) or not torch.cuda.is_current_stream_capturing()
+        return (hit is not None and hit[0].device == x.device) or not torch.cuda.is_current_stream_capturing()
 
     def _image_args(self, a, x, dt):
         """Image-row kernel: the tables and weight into the ``fovi_knnconv_args`` ``a``; returns

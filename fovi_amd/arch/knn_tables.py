@@ -555,25 +555,20 @@ def inverse_tables(slot_ptr, nbr_sorted, n_in, n_ref):
     ``(inv_ptr [n_in + 1] int32, inv [E] int32)``.
     """
     ptr = slot_ptr.numpy().astype(np.int64)
-    nbr = nbr_sorted.numpy().astype(np.int64)
+    nbr = nbr_sorted.numpy().astype(np.int64).reshape(-1)
     n_out = ptr.shape[0]
-    cnt = ptr & 0xFFFF
-    beg = ptr >> 16
-    # the slot of every list position: position j of output n is in slot v when beg <= j < beg + cnt
-    k = nbr.shape[1]
-    slot_of = np.full((n_out, k), -1, np.int64)
-    for v in range(n_ref):
-        j = np.arange(k)[None, :]
-        inside = (j >= beg[:, v:v + 1]) & (j < beg[:, v:v + 1] + cnt[:, v:v + 1])
-        slot_of = np.where(inside, v, slot_of)
-    valid = (nbr >= 0) & (nbr < n_in) & (slot_of >= 0)
-    ins = nbr[valid]
-    ent = (np.arange(n_out)[:, None] * n_ref + slot_of)[valid]
-    order = np.lexsort((ent, ins))
-    ins, ent = ins[order], ent[order]
-    inv_ptr = np.zeros(n_in + 1, np.int64)
-    np.add.at(inv_ptr, ins + 1, 1)
-    inv_ptr = np.cumsum(inv_ptr)
+    k = nbr_sorted.shape[1]
+    cnt = (ptr & 0xFFFF).reshape(-1)
+    # the list positions of every (output, slot) in turn: entry e's list begins at n k + begin
+    e = np.repeat(np.arange(n_out * n_ref, dtype=np.int64), cnt)
+    first = np.arange(n_out, dtype=np.int64)[:, None] * k + (ptr >> 16)
+    within = np.arange(e.size, dtype=np.int64) - np.repeat(np.cumsum(cnt) - cnt, cnt)
+    ins = nbr[first.reshape(-1)[e] + within]
+    valid = (ins >= 0) & (ins < n_in)
+    ins, e = ins[valid], e[valid]
+    key = np.sort(ins * (n_out * n_ref) + e)
+    ent = key % max(n_out * n_ref, 1)
+    inv_ptr = np.concatenate([[0], np.cumsum(np.bincount(ins, minlength=n_in))])
     return torch.from_numpy(inv_ptr.astype(np.int32)), torch.from_numpy(ent.astype(np.int32))
 
 
@@ -1317,6 +1312,12 @@ def spatial_order(coords, leaf=IMG_WINDOW):
     return torch.from_numpy(np.concatenate(out)).to(torch.int32)
 
 
+def _check_point_order(point_order, n):
+    """The C entry reads ``n`` int32 from it."""
+    if point_order is not None and (point_order.numel() != n or point_order.dtype != torch.int32):
+        raise ValueError(f"point_order must be {n} int32, got {point_order.numel()} {point_order.dtype}")
+
+
 def image_row_tables(slot_ptr, nbr_sorted, order, point_order, pp):
     """``(ent [G, V, pp, 4], points [G, pp], nact [G])`` (int32, host) of the image-row kernel:
     groups of ``pp`` output points with similar slot sets and the slots each group visits
@@ -1326,6 +1327,7 @@ def image_row_tables(slot_ptr, nbr_sorted, order, point_order, pp):
     slot_ptr, nbr_sorted = slot_ptr.cpu().contiguous(), nbr_sorted.cpu().contiguous()
     n, v = slot_ptr.shape
     k = nbr_sorted.shape[1]
+    _check_point_order(point_order, n)
     cap = sum(-(-min(IMG_WINDOW, n - w) // pp) for w in range(0, n, IMG_WINDOW))
     ent = torch.empty(cap, v, pp, 4, dtype=torch.int32)
     points = torch.empty(cap, pp, dtype=torch.int32)
@@ -1346,6 +1348,7 @@ def image_row_union(slot_ptr, point_order, pp):
     from .. import _lib
     slot_ptr = slot_ptr.cpu().contiguous()
     n, v = slot_ptr.shape
+    _check_point_order(point_order, n)
     windows = -(-n // IMG_WINDOW)
     mean = ctypes.c_double(0.0)
     got = _lib.load().fovi_knnconv_img_tables(_lib.ptr(slot_ptr), None, n, 1, v, None, _lib.ptr(point_order), pp,
