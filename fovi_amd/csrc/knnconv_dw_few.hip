@@ -12,8 +12,10 @@
 // A wave owns all rows o of a tile of up to 96 and a block of 32 columns, 32 / c_in slots x c_in
 // channels; for every point of its range it reads the slots' neighbour lists, one neighbour of every
 // slot per round (a slot without one reads a zero row), and skips a block none of whose slots has a
-// neighbour (not with a non-finite dy: its product with an empty slot's zero is NaN). Partial tiles
-// per point range go to a workspace and are added in range order.
+// neighbour. Partial tiles per point range go to a workspace and are added in range order.
+// With a non-finite dy (a flag its layout pass sets) the waves form every point's slot sums and multiply
+// those once, empty slots too, so that infinities and NaN come out as from the product of dy with
+// the matrix of slot sums: inf times an empty slot's zero is NaN, times a non-zero sum inf.
 // 128 images, 3 -> 96 channels, 4085 -> 964 points, k = 121 in V = 484 slots, x fp32: the slot-sum
 // matrix (717 MB) and an fp32 GEMM over it took 650 + 643 us; here 151 us, 32 us for the layouts and
 // 20 us for the reduction. Bound by the latency of the operand loads (two column blocks per wave, two
@@ -28,6 +30,21 @@ namespace {
 typedef uint32_t u32x4f __attribute__((ext_vector_type(4)));
 
 constexpr int DF_WAVES = 4;
+
+// Three bf16 parts of v, large to small, by truncation: they add up to v exactly; a non-finite v is
+// its own first part.
+__device__ __forceinline__ void split3(float v, uint16_t (&part)[3]) {
+  const uint32_t bits = __float_as_uint(v);
+  const float h = __uint_as_float(bits & 0xffff0000u);
+  const bool fin = (bits & 0x7f800000u) != 0x7f800000u;
+  const float r1 = fin ? v - h : 0.0f;
+  const float m = __uint_as_float(__float_as_uint(r1) & 0xffff0000u);
+  uint32_t hi = bits >> 16;
+  if (!fin && (bits & 0x007fffffu) && !(bits & 0x007f0000u)) hi |= 1u;   // NaN stays NaN
+  part[0] = static_cast<uint16_t>(hi);
+  part[1] = static_cast<uint16_t>(__float_as_uint(m) >> 16);
+  part[2] = static_cast<uint16_t>(__float_as_uint(r1 - m) >> 16);
+}
 
 // ---- operands with the images adjacent ------------------------------------------------------
 // out[((b / 16) * rows + fast * of + slow * os) * 16 + b % 16], `plane` elements apart for the parts;
@@ -70,17 +87,10 @@ __global__ __launch_bounds__(256) void images_adjacent_kernel(LayoutParams p, ui
         part[0][u >> 1] |= static_cast<uint32_t>(v) << sh;
         if (p.flag && (v & 0x7f80u) == 0x7f80u) *p.flag = 1;
       } else {
-        // by truncation: the parts add up to v exactly; a non-finite v is its own first part
-        const uint32_t bits = __float_as_uint(v);
-        const float h = __uint_as_float(bits & 0xffff0000u);
-        const bool fin = (bits & 0x7f800000u) != 0x7f800000u;
-        const float r1 = fin ? v - h : 0.0f;
-        const float m = __uint_as_float(__float_as_uint(r1) & 0xffff0000u);
-        uint32_t hi = bits >> 16;
-        if (!fin && (bits & 0x007fffffu) && !(bits & 0x007f0000u)) hi |= 1u;   // NaN stays NaN
-        part[0][u >> 1] |= hi << sh;
-        part[1][u >> 1] |= (__float_as_uint(m) >> 16) << sh;
-        part[NS - 1][u >> 1] |= (__float_as_uint(r1 - m) >> 16) << sh;
+        uint16_t t[3];
+        split3(v, t);
+#pragma unroll
+        for (int q = 0; q < NS; ++q) part[q][u >> 1] |= static_cast<uint32_t>(t[q]) << sh;
       }
     }
     uint16_t* o = p.out + ((b >> 4) * p.rows + f * p.of + s * p.os) * 16 + (b & 8);
@@ -122,7 +132,8 @@ __global__ __launch_bounds__(DF_WAVES * 64, 3) void knnconv_dw_few_kernel(DwFewP
   if (range >= ranges) return;
   const int o0 = blockIdx.y * MB * 32;
   if (ct >= p.n_ct) return;              // no barrier follows
-  const int n0 = range * p.per, n1 = min(p.Nout, n0 + p.per);
+  int n0 = range * p.per;
+  const int n1 = min(p.Nout, n0 + p.per);
 
   // this lane's column: slot v, channel c (columns past the slots: none)
   const int c = l32 % p.C, sl = l32 / p.C;
@@ -145,16 +156,64 @@ __global__ __launch_bounds__(DF_WAVES * 64, 3) void knnconv_dw_few_kernel(DwFewP
   auto row = [&](int n, int w, int r) {  // the slot's r-th neighbour, or the zero row
     return r < (w & 0xffff) ? p.nbr[static_cast<int64_t>(n) * p.K + (w >> 16) + r] : p.Nin;
   };
-  const bool every = *p.flag != 0;
   const int64_t dstep = static_cast<int64_t>(p.Nout) * p.Cout * 16, xstep = static_cast<int64_t>(p.Nin + 1) * p.C * 16;
   const int steps = p.bp / 16;
   struct Ops { bf16x8 a[MB], x[NS]; };
+  if (*p.flag != 0) {
+    // the slot sums (fp32, list order), then their parts; a zero part of a non-zero sum is replaced by
+    // the smallest normal number of its sign, so that no part turns inf * sum into NaN
+    for (int n = n0; n < n1; ++n) {
+      const int w = word(n);
+      const uint16_t* dn = p.dyt + static_cast<int64_t>(n) * p.Cout * 16;
+      for (int s = 0; s < steps; ++s) {
+        float sum[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) sum[u] = 0.0f;
+        for (int r = 0; __builtin_amdgcn_ballot_w64((w & 0xffff) > r) != 0; ++r) {
+          const uint16_t* xr = p.xt + (static_cast<int64_t>(row(n, w, r)) * p.C + c) * 16 + 8 * h + s * xstep;
+          float x[8];
+#pragma unroll
+          for (int q = 0; q < NS; ++q)
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {          // large parts first: exact
+              const float t = bf16_bits_to_f32(xr[q * p.plane + u]);
+              x[u] = q == 0 ? t : x[u] + t;
+            }
+#pragma unroll
+          for (int u = 0; u < 8; ++u) sum[u] += x[u];
+        }
+        bf16x8 xs[NS];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          if constexpr (NS == 1) {
+            xs[0][u] = static_cast<__bf16>(sum[u]);
+          } else {
+            uint16_t part[3];
+            split3(sum[u], part);
+#pragma unroll
+            for (int q = 0; q < NS; ++q) {
+              if ((part[q] & 0x7fffu) == 0u && sum[u] != 0.0f)
+                part[q] = 0x0080u | (__float_as_uint(sum[u]) >> 31 << 15);
+              xs[q][u] = __builtin_bit_cast(__bf16, part[q]);
+            }
+          }
+        }
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+          const bf16x8 a = *reinterpret_cast<const bf16x8*>(dn + s * dstep + oa[m]);
+#pragma unroll
+          for (int q = NS - 1; q >= 0; --q) acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, xs[q], acc[m], 0, 0, 0);
+        }
+      }
+    }
+    n0 = n1;
+  }
   int w = word(n0), i0 = n0 < n1 ? row(n0, w, 0) : p.Nin, wn = word(n0 + 1);
   for (int n = n0; n < n1; ++n) {
     // the next point's first neighbours, the one after's words
     const int inx = n + 1 < n1 ? row(n + 1, wn, 0) : p.Nin, wnn = word(n + 2);
     const uint16_t* dn = p.dyt + static_cast<int64_t>(n) * p.Cout * 16;
-    for (int r = 0; __builtin_amdgcn_ballot_w64((w & 0xffff) > r) != 0 || (every && r == 0); ++r) {
+    for (int r = 0; __builtin_amdgcn_ballot_w64((w & 0xffff) > r) != 0; ++r) {
       const int i = r == 0 ? i0 : row(n, w, r);
       const uint16_t* xr = p.xt + (static_cast<int64_t>(i) * p.C + c) * 16 + 8 * h;
       auto fetch = [&](Ops& t, int s) {

@@ -76,6 +76,41 @@ def test_autocast_training_step_takes_it_and_non_finite_gradients_show():
     assert torch.equal(torch.isfinite(bad), torch.isfinite(want))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("res_in,res_out,k,c_in,c_out,side,batch", [(12, 6, 25, 3, 96, 10, 9), (8, 8, 30, 4, 128, 3, 33),
+                                                                    (10, 8, 9, 1, 33, None, 5)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_non_finite_gradients_as_in_the_product_with_the_slot_sums(res_in, res_out, k, c_in, c_out, side, batch, dt):
+    """dW = dy^T a over the matrix a of slot sums (fp32; bf16 for a bf16 x): an infinite dy gives
+    infinities of the right sign, and NaN only where a is zero or infinities meet. x has values of few
+    significant bits (zero middle and low parts) beside ordinary ones, an infinity and a NaN. The values
+    that stay finite keep the fp32 sums' bound."""
+    layer = _layer(res_in, res_out, k, c_in, c_out, side)
+    n_in, n_out, v = layer.in_coords.shape[0], layer.out_coords.shape[0], layer.ref_coords.shape[0]
+    g = torch.Generator().manual_seed(8)
+    x = torch.randn(batch, c_in, n_in, generator=g).to(dt)
+    x[:, :, ::2] = x[:, :, ::2].bfloat16().to(dt)
+    x[0, 0, 1], x[1, 0, 2] = float("inf"), float("nan")
+    dy = torch.randn(batch, c_out, n_out, generator=g).bfloat16()
+    dy[2, 5, 3], dy[3, 6, 3], dy[4, 5, 7], dy[1, 7, 0] = (float(t) for t in ("inf", "-inf", "inf", "nan"))
+    got = layer._dw_few(x.cuda(), dy.cuda()).cpu()
+    sp, nbr = layer.slot_ptr.cpu().long(), layer.nbr_sorted.cpu().long()
+    a = torch.zeros(batch, c_in, n_out, v)
+    for r in range(int((sp & 0xFFFF).max())):            # in list order, as the slot-sum kernel
+        n, s = torch.nonzero((sp & 0xFFFF) > r, as_tuple=True)
+        a[:, :, n, s] += x[:, :, nbr[n, (sp[n, s] >> 16) + r]].float()
+    a = (a if dt == torch.float32 else a.bfloat16()).double()
+    want = torch.einsum("bon,bcnv->ocv", dy.double(), a).reshape(c_out, c_in * v)
+    if k == 30:
+        assert (torch.isinf(want[5]) & (want[5] > 0)).any() and (torch.isinf(want[6]) & (want[6] < 0)).any()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.isposinf(got), torch.isposinf(want))
+    assert torch.equal(torch.isneginf(got), torch.isneginf(want))
+    fin = torch.isfinite(want)
+    assert fin.any() and not fin.all()
+    assert_close_rel(got.double()[fin], want[fin], 1e-5, f"{dt}")
+
+
 def test_dw_few_sizes():
     lib = _lib.load()
     assert lib.fovi_knnconv_dw_few_workspace_bytes(128, 3, 96, 4085, 964, 484, _lib.F32) > 0
