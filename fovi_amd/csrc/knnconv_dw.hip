@@ -223,11 +223,12 @@ int launch_dw(const DwParams& p, int64_t total, int64_t padded, hipStream_t s) {
 // loads in flight per trip). A block takes one o and cc channels: a thread reads along c (the
 // partials' fast axis), the sums go through LDS and leave as runs of cc * V consecutive floats
 // (written straight from the reading order, one float per 4 V bytes, every line of dW is
-// touched V times).
-__global__ __launch_bounds__(256) void knnconv_dw_reduce_kernel(DwParams p, float* dw, int cc, int ccs) {
+// touched V times). Blocks along y take vt slots each; more than one of them only with cc = 1.
+__global__ __launch_bounds__(256) void knnconv_dw_reduce_kernel(DwParams p, float* dw, int cc, int ccs, int vt) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  float* out = reinterpret_cast<float*>(smem);                 // [cc][V]
-  const int V = static_cast<int>(p.V);
+  float* out = reinterpret_cast<float*>(smem);                 // [cc][V], V the block's slots
+  const int64_t vb = static_cast<int64_t>(blockIdx.y) * vt;
+  const int V = static_cast<int>(min(static_cast<int64_t>(vt), p.V - vb));
   const int64_t nc = (p.C + cc - 1) / cc;
   const int64_t o = blockIdx.x / nc, c0 = (blockIdx.x % nc) * cc;
   const int lc = threadIdx.x & (cc - 1), v0 = threadIdx.x >> ccs, dv = 256 >> ccs;
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(256) void knnconv_dw_reduce_kernel(DwParams p, floa
   const int64_t stride = p.V * p.tiles_o * p.tiles_c * (p.to * p.tc);   // next (group, chunk)
   if (c < p.C) {
     const int64_t tile = (o / p.to) * p.tiles_c + c / p.tc;
-    const float* base = p.part + tile * (p.to * p.tc) + (o % p.to) * p.tc + c % p.tc;
+    const float* base = p.part + (vb * p.tiles_o * p.tiles_c + tile) * (p.to * p.tc) + (o % p.to) * p.tc + c % p.tc;
     for (int v = v0; v < V; v += dv) {
       const float* src = base + v * p.tiles_o * p.tiles_c * (p.to * p.tc);
       float sum = 0.0f;
@@ -255,7 +256,7 @@ __global__ __launch_bounds__(256) void knnconv_dw_reduce_kernel(DwParams p, floa
   __syncthreads();
   const int64_t left = p.C - c0;
   const int count = static_cast<int>(left < cc ? left : cc) * V;
-  float* dst = dw + (o * p.C + c0) * p.V;
+  float* dst = dw + (o * p.C + c0) * p.V + vb;
   for (int i = threadIdx.x; i < count; i += 256) dst[i] = out[i];
 }
 
@@ -316,20 +317,19 @@ extern "C" int fovi_knnconv_dw(const fovi_knnconv_dw_args* a, void* stream) {
   const int rc = p.to == 256 ? (p.tc == 256 ? launch_dw<256, 256>(p, total, padded, s) : launch_dw<256, 128>(p, total, padded, s))
                              : (p.tc == 256 ? launch_dw<128, 256>(p, total, padded, s) : launch_dw<128, 128>(p, total, padded, s));
   if (rc) return rc;
-  // channels per reduction block: 32, fewer where their V sums pass 64 KB of LDS
+  // channels per reduction block: 32, fewer where their V sums pass 64 KB of LDS; slots in pieces where
+  // one channel's do
+  constexpr int64_t sums = 64 * 1024 / 4;
   int ccs = 5;
-  while (ccs > 0 && (p.V << ccs) * 4 > 64 * 1024) --ccs;
-  const int64_t lds = (p.V << ccs) * 4, blocks = p.Cout * ((p.C + (1 << ccs) - 1) >> ccs);
-  if (lds > 160 * 1024 || blocks > 0x7fffffff) {
-    set_error("fovi_knnconv_dw: n_ref=%lld too large", (long long)p.V);
+  while (ccs > 0 && (p.V << ccs) > sums) --ccs;
+  const int64_t vt = p.V < sums ? p.V : sums, pieces = (p.V + vt - 1) / vt;
+  const int64_t blocks = p.Cout * ((p.C + (1 << ccs) - 1) >> ccs);
+  if (blocks > 0x7fffffff || pieces > 65535) {
+    set_error("fovi_knnconv_dw: c_out=%lld x c_in=%lld x n_ref=%lld too large", (long long)p.Cout, (long long)p.C,
+              (long long)p.V);
     return 1;
   }
-  if (lds > 64 * 1024 &&
-      reserve_dynamic_lds(reinterpret_cast<const void*>(&knnconv_dw_reduce_kernel), static_cast<size_t>(lds)) != hipSuccess) {
-    set_error("fovi_knnconv_dw: cannot reserve %lld bytes of LDS", (long long)lds);
-    return 1;
-  }
-  hipLaunchKernelGGL(knnconv_dw_reduce_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), static_cast<size_t>(lds),
-                     s, p, a->dw, 1 << ccs, ccs);
+  hipLaunchKernelGGL(knnconv_dw_reduce_kernel, dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(pieces)), dim3(256),
+                     static_cast<size_t>((vt << ccs) * 4), s, p, a->dw, 1 << ccs, ccs, static_cast<int>(vt));
   return check_launch("fovi_knnconv_dw(reduce)");
 }
