@@ -14,7 +14,7 @@ import torch
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libfovi_hip.so")
 
-ABI_VERSION = 35
+ABI_VERSION = 36
 F32, BF16, F8E4M3 = 0, 1, 2
 NEAREST, BILINEAR = 0, 1
 PAD_ZEROS, PAD_BORDER = 0, 1
@@ -32,7 +32,7 @@ EXPORTED = ("fovi_abi_version", "fovi_last_error", "fovi_sampler_fwd", "fovi_knn
             "fovi_knnconv_dw", "fovi_knnpool_bwd", "fovi_knnconv_last_path",
             "fovi_knnconv_fwd_noalloc", "fovi_knnconv_wide_tiles", "fovi_knnconv_weight_img_elems",
             "fovi_knnconv_pack_weight_img", "fovi_knnconv_img_tables", "fovi_knnconv_dw_few",
-            "fovi_knnconv_dw_few_workspace_bytes")
+            "fovi_knnconv_dw_few_workspace_bytes", "fovi_knnconv_dw_few_us")
 
 
 class SamplerArgs(C.Structure):
@@ -265,6 +265,8 @@ def load(path: str = LIB_PATH):
     lib.fovi_knnconv_dw.restype = C.c_int
     lib.fovi_knnconv_dw_few_workspace_bytes.argtypes = [C.c_int64] * 6 + [C.c_int32]
     lib.fovi_knnconv_dw_few_workspace_bytes.restype = C.c_int64
+    lib.fovi_knnconv_dw_few_us.argtypes = [C.c_int64] * 6 + [C.c_int32, C.c_double]
+    lib.fovi_knnconv_dw_few_us.restype = C.c_double
     lib.fovi_knnconv_dw_few.argtypes = [C.POINTER(KnnConvDwFewArgs), C.c_void_p]
     lib.fovi_knnconv_dw_few.restype = C.c_int
     lib.fovi_knnpool_bwd.argtypes = [C.POINTER(KnnPoolBwdArgs), C.c_void_p]

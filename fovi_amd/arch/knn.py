@@ -30,7 +30,7 @@ forward of the transposed layer (``_TransposedKnnConv``, over the inverse
 neighbour table, no atomics). ``dW`` of bf16 layers runs over each slot's
 (output, input) pairs (``fovi_knnconv_dw``), that of layers of at most 8
 channels with a bf16 output gradient over the images
-(``fovi_knnconv_dw_few``); the others take the slot sums again
+(``fovi_knnconv_dw_few``) where that pays; the others take the slot sums again
 (``fovi_knnconv_slotsum``) and a library GEMM. The fp8 path has no backward.
 """
 from __future__ import annotations
@@ -623,6 +623,7 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
     # (class defaults: a layer unpickled from a file without these attributes runs the other kernels)
     image_rows = False
     _img = None
+    _few_lists = None
 
     def _image_plan(self, batch):
         """``(work, (rows per workgroup / 32, images per point, 32-column blocks per wave))`` of the
@@ -949,7 +950,8 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         bsz, c, n_in = x.shape
         n_out, v, c_out = self.out_coords.shape[0], self.ref_coords.shape[0], self.out_channels
         dt = x.dtype
-        dw_few = self._dw_few(x, dy) if need_w and self.dw_fused and dy.dtype == torch.bfloat16 and c <= 8 else None
+        dw_few = (self._dw_few(x, dy) if need_w and self.dw_fused and dy.dtype == torch.bfloat16 and c <= 8
+                  and self._dw_few_pays(x) else None)
         if dw_few is not None and not need_x:
             return None, dw_few.to(weight.dtype)
         dy = dy.to(dt)
@@ -999,6 +1001,46 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         return (dt == torch.bfloat16 and self.in_channels % 8 == 0 and self.out_channels % 8 == 0
                 and x.stride(1) == 1 and x.stride(2) % 8 == 0 and x.stride(0) % 8 == 0
                 and x.data_ptr() % 16 == 0)
+
+    def _dw_few_pays(self, x):
+        """Whether ``fovi_knnconv_dw_few`` is expected to be the fastest weight gradient of ``x``: its
+        estimate (whole steps of 16 images, so few images pay for 16) against that of the pair
+        lists, where they apply, or of the slot sums and the GEMM; up to 30 us it is taken
+        anyway, since the GEMM path's launches alone take the host 45 us. Both sides of 5288 calls
+        measured (1 to 8 channels, 8 to 384 outputs, V = 9 to 484, 1 to 128 images): time lost to
+        the better choice 3% in all; always taking it 11%, and up to 8 times as slow for
+        one image (fp32, 3 -> 384 channels, 2500 points, V = 196: 209 against 43 us). 128 images 3 -> 96,
+        964 points, V = 484: 203 against 1290 us."""
+        bsz, c, n_in = x.shape
+        n_out, v, c_out = self.out_coords.shape[0], self.ref_coords.shape[0], self.out_channels
+        code = _lib.dtype_code(x.dtype)
+        lib = _lib.load()
+        if lib.fovi_knnconv_dw_few_workspace_bytes(bsz, c, c_out, n_in, n_out, v, code) < 0:
+            return False
+        rounds, entries = self._few_channel_lists()
+        few = lib.fovi_knnconv_dw_few_us(bsz, c, c_out, n_in, n_out, v, code, rounds)
+        if self._dw_fused_ok(x, x.dtype):
+            return few < self._dw_split_time(bsz, -(-n_out // self.dw_chunk) * v)[0]
+        size, rows = x.element_size(), bsz * n_out
+        mb = rows * size * 1e-6
+        gflop = 2e-9 * rows * v * c * c_out
+        if x.dtype == torch.float32:
+            other = 19 + mb * (0.45 * v * c + entries * c + 1.1 * c_out) + 9.4 * gflop + 2.2e-3 * rows
+        else:
+            other = 20 + mb * (v * c + 1.9 * entries * c + 3.4 * c_out) + 2.5 * gflop + 1.1e-3 * rows
+        return few < max(other, 30.0)
+
+    def _few_channel_lists(self):
+        """``(rounds, entries)``: the mean neighbour count of the fullest slot of a block of
+        ``32 // c_in`` slots, for the block where it is largest, and the mean list length of a
+        point (from about 256 points, once)."""
+        if self._few_lists is None:
+            ptr = self.slot_ptr.cpu() if self._img is None else self._img.slot_ptr
+            cnt = (ptr[::max(1, len(ptr) // 256)] & 0xFFFF).to(torch.float32)
+            slots = 32 // self.in_channels
+            blocks = F.pad(cnt, (0, -cnt.shape[1] % slots)).unflatten(1, (-1, slots)).amax(2)
+            self._few_lists = (float(blocks.mean(0).max()), float(cnt.sum(1).mean()))
+        return self._few_lists
 
     def _dw_few(self, x, dy):
         """``dW`` (fp32, reference layout) of a layer with at most 8 input channels from a bf16 ``dy`` of
@@ -1051,7 +1093,11 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         return dw
 
     def _dw_split(self, batch, segments):
-        """Images per workgroup of ``fovi_knnconv_dw``: the split with the least estimated time. More
+        """Images per workgroup of ``fovi_knnconv_dw``."""
+        return self._dw_split_time(batch, segments)[1]
+
+    def _dw_split_time(self, batch, segments):
+        """``(us, images per workgroup)`` of ``fovi_knnconv_dw`` at the split with the least estimated time. More
         groups fill the chip more evenly (one workgroup per CU with 256 x 256 channel tiles,
         two or more with smaller ones), but each writes a partial tile of every slot, which is
         read again: one group per image cost 96 -> 256 channels with V = 100 at 256 images
@@ -1075,7 +1121,7 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
             if best is None or t < best[0]:
                 best = (t, ipg)
             groups = max(groups + 1, groups * 9 // 8)
-        return best[1]
+        return best
 
     def _slot_pairs(self, device):
         """``knn_tables.slot_pairs`` of this layer, built on the first backward and kept."""

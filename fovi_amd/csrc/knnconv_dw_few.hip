@@ -20,6 +20,7 @@
 // matrix (717 MB) and an fp32 GEMM over it took 650 + 643 us; here 151 us, 32 us for the layouts and
 // 20 us for the reduction. Bound by the latency of the operand loads (two column blocks per wave, two
 // waves per SIMD and no load ahead: 227 us).
+#include <cmath>
 #include <type_traits>
 
 #include "common.h"
@@ -297,10 +298,15 @@ bool few_plan(int64_t B, int64_t C, int64_t Cout, int64_t Nin, int64_t Nout, int
   const int64_t row_blocks = (Cout + 31) / 32;
   f.o_tiles = static_cast<int>((row_blocks + 2) / 3);
   f.mb = static_cast<int>((row_blocks + f.o_tiles - 1) / f.o_tiles);
-  // point ranges: about 3072 waves in all (three per SIMD), each range at least one point
+  // point ranges: about 3072 waves in all (three per SIMD), each range at least one point. A wave's
+  // chain takes about a microsecond per point and step of 16 images, the reduction's 75 ns per range
+  // (eight loads in flight), so their sum is least at sqrt(13 steps points) ranges: more only
+  // lengthen the reduction (1156 points, 8 images, one tile: 89 us with 1156 ranges, 40 with 122).
   const int64_t tiles = static_cast<int64_t>(f.n_ct) * f.o_tiles;
   int64_t ranges = 3072 / tiles > 0 ? 3072 / tiles : 1;
   if (ranges > Nout) ranges = Nout;
+  const double chain = std::sqrt(13.0 * static_cast<double>(f.bp / 16) * static_cast<double>(Nout));
+  if (ranges > chain) ranges = static_cast<int64_t>(chain);
   const int64_t per = (Nout + ranges - 1) / ranges;
   f.per = static_cast<int>(per);
   f.ranges = static_cast<int>((Nout + per - 1) / per);
@@ -345,6 +351,20 @@ extern "C" int64_t fovi_knnconv_dw_few_workspace_bytes(int64_t batch, int64_t c_
   fovi::FewPlan f;
   if (!fovi::few_plan(batch, c_in, c_out, n_in, n_out, n_ref, x_dtype, f)) return -1;
   return (f.dyt + f.parts * f.xt) * 2 + f.part * 4 + 16;
+}
+
+// Microseconds on the plan above, fitted to 5288 calls (1 to 8 channels, 8 to 384 outputs, 4 to 16384
+// points, V = 9 to 484, 1 to 128 images; estimate / time: 0.65 to 1.3 for 98% of them): launches, a wave's
+// chain over its points, the layout passes (0.6 us per MB read and written), the partial tiles.
+extern "C" double fovi_knnconv_dw_few_us(int64_t batch, int64_t c_in, int64_t c_out, int64_t n_in, int64_t n_out,
+                                         int64_t n_ref, int32_t x_dtype, double rounds) {
+  fovi::FewPlan f;
+  if (!fovi::few_plan(batch, c_in, c_out, n_in, n_out, n_ref, x_dtype, f)) return -1.0;
+  const double chain = f.per * rounds, steps = static_cast<double>(f.bp / 16);
+  const double layout = static_cast<double>(n_out) * c_out * (batch + f.bp) * 2 +
+                        static_cast<double>(n_in) * c_in * ((f.parts == 3 ? 4 : 2) * batch + 2 * f.parts * f.bp);
+  return 15.0 + 0.2 * chain + (f.parts == 3 ? 0.65 : 0.45) * chain * steps + 0.6e-6 * layout +
+         0.43e-6 * static_cast<double>(f.part) * 8 + 0.02 * f.ranges;
 }
 
 extern "C" int fovi_knnconv_dw_few(const fovi_knnconv_dw_few_args* a, void* stream) {

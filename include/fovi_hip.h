@@ -23,7 +23,7 @@
 extern "C" {
 #endif
 
-#define FOVI_ABI_VERSION 35
+#define FOVI_ABI_VERSION 36
 
 enum fovi_dtype { FOVI_F32 = 0, FOVI_BF16 = 1, FOVI_F8E4M3 = 2 };
 enum fovi_interp { FOVI_NEAREST = 0, FOVI_BILINEAR = 1 };
@@ -742,6 +742,11 @@ typedef struct fovi_knnconv_dw_few_args {
 int64_t fovi_knnconv_dw_few_workspace_bytes(int64_t batch, int64_t c_in, int64_t c_out, int64_t n_in, int64_t n_out,
                                             int64_t n_ref, int32_t x_dtype);
 int fovi_knnconv_dw_few(const fovi_knnconv_dw_few_args* args, void* stream);
+/* Its estimated time in microseconds (-1 for sizes it does not take); rounds: the neighbours of the
+ * fullest slot of a column block (32 / c_in consecutive slots), averaged over the points, for the
+ * block where that is largest. */
+double fovi_knnconv_dw_few_us(int64_t batch, int64_t c_in, int64_t c_out, int64_t n_in, int64_t n_out, int64_t n_ref,
+                              int32_t x_dtype, double rounds);
 
 #ifdef __cplusplus
 }

@@ -118,3 +118,35 @@ def test_dw_few_sizes():
         assert lib.fovi_knnconv_dw_few_workspace_bytes(*args) == -1
     assert lib.fovi_knnconv_dw_few(_lib.KnnConvDwFewArgs(), None) != 0
     assert b"null pointer" in lib.fovi_last_error()
+
+
+def test_dw_few_is_taken_where_it_pays():
+    """Few images of a large layer are padded to 16: slot sums and a GEMM are faster there."""
+    layer = _layer(48, 24, 49, 3, 96, 14, device="cpu")
+    n_in = layer.in_coords.shape[0]
+    for dt in (torch.float32, torch.bfloat16):
+        pays = [layer._dw_few_pays(torch.zeros(b, 3, n_in, dtype=dt)) for b in (1, 2, 128)]
+        assert pays == [False, False, True]
+    small = _layer(8, 4, 9, 3, 32, None, device="cpu")          # below the host's own time
+    assert small._dw_few_pays(torch.zeros(1, 3, small.in_coords.shape[0]))
+    eight = _layer(48, 24, 49, 8, 96, 14, device="cpu")         # channels-last bf16: the pair lists
+    rows = lambda b: torch.zeros(b, eight.in_coords.shape[0], 8, dtype=torch.bfloat16).transpose(1, 2)
+    assert not eight._dw_few_pays(rows(1)) and eight._dw_few_pays(rows(128))
+    lib = _lib.load()
+    assert lib.fovi_knnconv_dw_few_us(8, 9, 96, 4, 4, 9, _lib.F32, 1.0) == -1.0
+    assert lib.fovi_knnconv_dw_few_us(128, 3, 96, 4085, 964, 484, _lib.F32, 2.0) > 100.0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,few", [(1, False), (2, False), (128, True)])
+def test_the_backward_follows_the_rule(batch, few, monkeypatch):
+    layer = _layer(48, 24, 49, 3, 96, 14)
+    g = torch.Generator().manual_seed(9)
+    x = torch.randn(batch, 3, layer.in_coords.shape[0], generator=g)
+    dy = torch.randn(batch, 96, layer.out_coords.shape[0], generator=g).bfloat16()
+    calls = []
+    inner = layer._dw_few
+    monkeypatch.setattr(layer, "_dw_few", lambda *a: calls.append(1) or inner(*a))
+    _, dw = layer._backward(x.cuda(), layer.weight, dy.cuda(), False, True)
+    assert bool(calls) == few
+    assert_close_rel(dw.double().cpu(), _dw64(layer, x, dy), 1e-5, f"{batch}")
