@@ -756,15 +756,21 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         return frag, flag, w_scale, ent, points, nact
 
     @staticmethod
-    def _image_input(x, dt):
-        """``x`` as channels-last rows of a multiple of 16 bytes, 128 images within 2 GiB (``x``
-        itself where it is)."""
+    def _image_input_ready(x, dt):
+        """Whether ``x`` is channels-last rows of a multiple of 16 bytes, 128 images within 2 GiB."""
         al = 16 // dt.itemsize
         b, c, n = x.shape
-        if (c % al == 0 and x.stride(1) == 1 and x.stride(2) % al == 0 and x.stride(0) % al == 0
+        return (c % al == 0 and x.stride(1) == 1 and x.stride(2) % al == 0 and x.stride(0) % al == 0
                 and x.data_ptr() % 16 == 0
-                and ((min(b, 128) - 1) * x.stride(0) + (n - 1) * x.stride(2) + c) * dt.itemsize < 2 ** 31 - 4096):
+                and ((min(b, 128) - 1) * x.stride(0) + (n - 1) * x.stride(2) + c) * dt.itemsize < 2 ** 31 - 4096)
+
+    @staticmethod
+    def _image_input(x, dt):
+        """``x`` as the image-row kernel reads it (``x`` itself where it is that already)."""
+        if KNNConvLayer._image_input_ready(x, dt):
             return x
+        al = 16 // dt.itemsize
+        b, c, n = x.shape
         cp = -(-c // al) * al
         buf = (torch.empty if cp == c else torch.zeros)(b, n, cp, dtype=dt, device=x.device)
         buf[:, :, :c].copy_(x.transpose(1, 2))
@@ -1178,8 +1184,8 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
                              f"got {tuple(x.shape)}")
         if self.tile_lo is None:
             raise NotImplementedError("fp8 kNN-conv needs the tile tables (k <= 255, tile spans <= 65535)")
-        image = (self._image_path(x, torch.float8_e4m3fn) and self.in_channels % 64 == 0
-                 and self._image_input(x, torch.float8_e4m3fn) is x)
+        image = (self.in_channels % 64 == 0 and self._image_input_ready(x, torch.float8_e4m3fn)
+                 and self._image_path(x, torch.float8_e4m3fn))
         mfma = not image and self._mfma_path(x, torch.float8_e4m3fn)
         self.last_weight_layout = "image" if image else "mfma" if mfma else "rows"
         if image:

@@ -221,3 +221,42 @@ def test_gradients_through_the_image_row_kernel(dt):
     tol = 2e-5 if dt == torch.float32 else 1e-2
     for a, b, what in zip(got, want, ("dx", "dW", "db")):
         assert_close_rel(a.cpu(), b.cpu(), tol, what)
+
+
+def test_input_layouts_the_kernel_reads():
+    buf = torch.zeros(2, 9, 96, dtype=torch.uint8).view(torch.float8_e4m3fn)
+    e4m3 = torch.float8_e4m3fn
+    ready = KNNConvLayer._image_input_ready
+    assert ready(buf[:, :, :64].transpose(1, 2), e4m3) and ready(buf[:, :, 16:80].transpose(1, 2), e4m3)
+    assert not ready(buf[:, :, 8:72].transpose(1, 2), e4m3)         # rows not 16-byte aligned
+    assert not ready(buf[:, :, :56].transpose(1, 2), e4m3)          # rows not a multiple of 16 bytes
+    assert not ready(buf[:, :, :64].permute(0, 2, 1).contiguous(), e4m3)
+    x = torch.zeros(2, 9, 12).transpose(1, 2)
+    assert KNNConvLayer._image_input(x, torch.float32) is x
+
+
+@pytest.mark.gpu
+def test_unaligned_e4m3_rows_are_not_copied(monkeypatch):
+    """They run the kernels that read them as they are: the answer, or the refusal, of those."""
+    layer = _layer(16, 16, 9, 64, 256)
+    x = torch.randn(9, 64, 256, generator=torch.Generator().manual_seed(9)).bfloat16().cuda()
+    xq = layer.quantize_input(x)
+    want = layer(xq)
+    assert layer.last_weight_layout == "image"
+
+    def never(*a):
+        raise AssertionError("copied")
+    monkeypatch.setattr(KNNConvLayer, "_image_input", staticmethod(never))
+    buf = torch.zeros(9, 256, 96, dtype=torch.uint8, device="cuda").view(torch.float8_e4m3fn)
+    buf.view(torch.uint8)[:, :, 8:72] = xq.data.view(torch.uint8).transpose(1, 2)
+    xq = xq._replace(data=buf[:, :, 8:72].transpose(1, 2))
+    try:
+        got = layer(xq)
+    except RuntimeError as e:
+        assert "fovi_knnconv_fwd" in str(e)
+        layer.image_rows = False
+        with pytest.raises(RuntimeError, match="fovi_knnconv_fwd"):
+            layer(xq)
+        return
+    assert layer.last_weight_layout != "image"
+    assert_close_rel(got.float().cpu(), want.float().cpu(), 1e-2, "unaligned")
