@@ -58,7 +58,12 @@ __all__ = [
     "register_with_reference",
 ]
 
-# Smallest batch and fewest input channels of the image-row kernel.
+# Smallest batch and fewest input channels of the image-row kernel. From 8 images and 16 channels on
+# it was at most 8% slower, and in the mean 3 to 11 times as fast, than each of the kernels whose
+# tiles are points of one image (row-packed, generic, vector units) on 4901 layers of 16 to 384 ->
+# 8 to 384 channels, V = 4 to 196. With 1 to 7 images most layers would gain as well (6.2 times in
+# the mean), but wide ones can lose (2 images, 9604 points, 256 -> 384, V = 9: 265 against 92 us):
+# those batches keep the kernels they had.
 IMG_MIN_BATCH = 8
 IMG_MIN_CHANNELS = 16
 
@@ -164,8 +169,9 @@ class KNNBaseLayer:
 
 
 class _KnnConvFn(torch.autograd.Function):
-    """Forward ``fovi_knnconv_fwd``; backward = the slot sums again (``fovi_knnconv_slotsum``)
-    and the transposed gather (``fovi_knnconv_bwd_x``) around two library GEMMs."""
+    """Forward ``fovi_knnconv_fwd``; backward ``KNNConvLayer._backward``: the input gradient as the
+    forward of the transposed layer, the weight gradient by pair lists (bf16), over the images
+    (few channels, bf16 ``dy``) or by the slot sums and a library GEMM."""
 
     @staticmethod
     def forward(ctx, x, layer, weight, bias, activation=None):
@@ -715,8 +721,8 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         return packed
 
     def _image_path(self, x, dt):
-        """Whether this call runs the image-row kernel: a batch of at least ``IMG_MIN_BATCH`` (below,
-        most of a block of 16 images would be padding), at least ``IMG_MIN_CHANNELS`` input channels,
+        """Whether this call runs the image-row kernel: a batch of at least ``IMG_MIN_BATCH``, at least
+        ``IMG_MIN_CHANNELS`` input channels,
         32-bit offsets within a block of images, and less estimated work than the wide-layer
         kernel where that one applies. The choice depends on the layer and the call alone, not on
         earlier calls (but for a layer unpickled without its tables: their upload cannot be
@@ -731,7 +737,9 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
             # CU; its time in slots of the image-row kernel, from both sides at V = 9 and 25,
             # 256 to 16384 points, 8 to 256 images (V = 9, 16384 points, B = 64: bf16 0.78 against
             # 0.62 ms, e4m3 0.64 against 0.39; V = 25: 3.15 against 2.80 and 2.36 against 1.54; the
-            # same with 24 images in two blocks of 16: 1.20 against 1.32, bf16)
+            # same with 24 images in two blocks of 16: 1.20 against 1.32, bf16). Used beyond: on 1632
+            # wide layers, V = 4 to 196, the choice costs 1.7% over the best in all;
+            # image rows over 10% slower twice (e4m3, V = 4), the wide kernel 34 times
             tiles = bsz * -(-self.out_coords.shape[0] // 256) * -(-self.out_channels // 256)
             pad = -(-self.out_coords.shape[0] // 256) * 256 / self.out_coords.shape[0]
             v = self.ref_coords.shape[0]

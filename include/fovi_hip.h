@@ -396,12 +396,12 @@ int fovi_knnconv_pack_weight_img(const float* w_ref, int64_t c_out, int64_t c_in
 /*
  * Host tables of the image-row kernel (all pointers host memory): groups of pp output points
  * with similar slot sets, formed within windows of `window` consecutive points of point_order (a
- * permutation of the points, or NULL: the index order). Writes, per
- * group, its points (-1: none), the number of slots its points use, and n_ref * pp entries of 4 words
- * {neighbour 1, neighbour 2 (0x80000000: none), count << 16 | begin, position} with the used slots first, each part in visit order. Returns the number of groups (at most
- * (n_out / window + 1) * ceil(window / pp)), -1 on bad arguments. With ent NULL nothing is
- * written and only every stride-th window is grouped; *mean_union (optional) gets the mean number
- * of used slots per group.
+ * permutation of the points, or NULL: the index order). Writes, per group, its points (-1: none),
+ * the number of slots its points use, and n_ref * pp entries of 4 words {neighbour 1, neighbour 2
+ * (0x80000000: none), count << 16 | begin, position} with the used slots first, each part in visit
+ * order. Returns the number of groups (at most (n_out / window + 1) * ceil(window / pp)), -1 on bad
+ * arguments or where memory runs out. With ent NULL nothing is written and only every stride-th
+ * window is grouped; *mean_union (optional) gets the mean number of used slots per group.
  */
 int64_t fovi_knnconv_img_tables(const int32_t* slot_ptr, const int32_t* nbr, int64_t n_out, int64_t k, int64_t n_ref,
                                 const int32_t* slot_order, const int32_t* point_order, int32_t pp, int64_t window,
@@ -690,13 +690,13 @@ int fovi_local_rf_slots(const fovi_local_rf_args* args, void* stream);
  * fp32 accumulation of bf16 products, fp32 output in the reference weight
  * layout. pairs holds (n, i) int32 pairs in n_chunks * n_ref segments,
  * segment q * n_ref + v at [pair_off[q * n_ref + v], pair_off[q * n_ref + v + 1])
- * holding slot v's pairs of one chunk of output points (the layer: 256
- * consecutive points per chunk, output order), optionally padded with
- * (-1, -1) entries (the layer pads to multiples of 64, the kernel's step). One workgroup takes one segment for
+ * holding slot v's pairs of one chunk of output points (the layer: all of
+ * them, output order), optionally padded with (-1, -1) entries (the layer
+ * pads to multiples of 64). One workgroup takes one segment for
  * images_per_group consecutive images; the workspace holds its partial tile
- * (fovi_knnconv_dw_workspace_bytes). x and
- * dy bf16 channels-last (element strides [batch, channel, point] with channel
- * stride 1, rows 16-byte aligned); c_in and c_out multiples of 8.
+ * (fovi_knnconv_dw_workspace_bytes). x and dy bf16 channels-last (element
+ * strides [batch, channel, point] with channel stride 1, rows 16-byte
+ * aligned); c_in and c_out multiples of 8.
  */
 typedef struct fovi_knnconv_dw_args {
   const void* x;              /* bf16 [batch, c_in, n_in] (strides below) */
@@ -722,7 +722,8 @@ int fovi_knnconv_dw(const fovi_knnconv_dw_args* args, void* stream);
  * any element strides [batch, channel, point]; fp32 x enters as three bf16 parts that add up to it
  * exactly. slot_ptr [n_out, n_ref] and nbr_sorted [n_out, k] are the forward's tables. The
  * workspace (fovi_knnconv_dw_few_workspace_bytes, -1 for sizes it does not take; 16-byte
- * aligned) holds both operands with the images adjacent and the partial sums.
+ * aligned) holds both operands with the images adjacent and the partial sums. Infinities and NaN
+ * come out as from the product of dy with the matrix of slot sums.
  */
 typedef struct fovi_knnconv_dw_few_args {
   const void* x;
