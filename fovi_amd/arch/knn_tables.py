@@ -1329,10 +1329,10 @@ def image_row_tables(slot_ptr, nbr_sorted, order, point_order, pp):
     k = nbr_sorted.shape[1]
     _check_point_order(point_order, n)
     cap = sum(-(-min(IMG_WINDOW, n - w) // pp) for w in range(0, n, IMG_WINDOW))
-    ent = torch.empty(cap, v, pp, 4, dtype=torch.int32)
-    points = torch.empty(cap, pp, dtype=torch.int32)
-    nact = torch.empty(cap, dtype=torch.int32)
-    ordt = None if order is None else torch.tensor(list(order), dtype=torch.int32)
+    ent = torch.empty(cap, v, pp, 4, dtype=torch.int32, device="cpu")
+    points = torch.empty(cap, pp, dtype=torch.int32, device="cpu")
+    nact = torch.empty(cap, dtype=torch.int32, device="cpu")
+    ordt = None if order is None else torch.tensor(list(order), dtype=torch.int32, device="cpu")
     got = _lib.load().fovi_knnconv_img_tables(_lib.ptr(slot_ptr), _lib.ptr(nbr_sorted), n, k, v, _lib.ptr(ordt),
                                               _lib.ptr(point_order), pp, IMG_WINDOW, 1, _lib.ptr(ent),
                                               _lib.ptr(points), _lib.ptr(nact), None)

@@ -152,7 +152,7 @@ class GridSampler(BaseGridSampler):
                 raise ValueError(f"view_image entries must be in [0, {n_img})")
         elif n_views > n_img:
             raise ValueError(f"{n_views} views of {n_img} images need a view_image map")
-        host = torch.empty(n_views * 7, dtype=torch.int32, pin_memory=cuda)
+        host = torch.empty(n_views * 7, dtype=torch.int32, device="cpu", pin_memory=cuda)
         host[:4 * n_views].view(torch.float64).copy_(half.reshape(-1))
         host[4 * n_views:6 * n_views].view(torch.float32).copy_(fix_loc.reshape(-1))
         if vi is not None:
