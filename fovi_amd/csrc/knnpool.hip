@@ -382,12 +382,13 @@ static void launch_pool(const PoolParams& p, hipStream_t s) {
   }
   const int64_t total = p.B * p.Nout * p.C;
   // planes: enough points for a wave's lanes to share a plane row (below 16 the channels are the
-  // better lanes: the last average pooling has one output point)
+  // better lanes: the last average pooling has one output point). The kernel reads input 0 for a
+  // neighbour it does not have, so there must be one.
   const int64_t cgroups = (p.C + PL_U - 1) / PL_U;
   const int ls = plane_lanes(p.Nout);
   const int64_t n_tiles = (p.Nout + (int64_t(1) << ls) - 1) >> ls;
   const int64_t pblocks = n_tiles * ((p.B * cgroups + (256 >> ls) - 1) / (256 >> ls));
-  if (p.xs2 == 1 && p.K <= POOL_KF && p.Nout >= 16 && p.B * cgroups <= 0x7fffffffLL && pblocks <= 0x7fffffffLL) {
+  if (p.xs2 == 1 && p.K <= POOL_KF && p.Nout >= 16 && p.Nin > 0 && p.B * cgroups <= 0x7fffffffLL && pblocks <= 0x7fffffffLL) {
     const auto args = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(pblocks)), dim3(256), 0, s, p, ls,
                          static_cast<uint32_t>(n_tiles), static_cast<uint32_t>(cgroups),

@@ -4,6 +4,7 @@ stride 2 of the same values takes the latter."""
 import pytest
 import torch
 
+from fovi_amd import _lib
 from fovi_amd.arch.knn import KNNPoolingLayer
 from fovi_amd.sensing.coords import SamplingCoords
 
@@ -43,3 +44,21 @@ def test_planes_equal_the_any_stride_kernels(mode, dt, res_in, res_out, k, c, ba
         dx = layer._backward(x, d)
         assert dx.stride(2) == 1
         assert torch.equal(dx.nan_to_num(7.0), ref.nan_to_num(7.0)) and torch.equal(dx.isnan(), ref.isnan())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode,want", [(_lib.POOL_MAX, float("-inf")), (_lib.POOL_AVG, float("nan")),
+                                       (_lib.POOL_SUM, 0.0), (_lib.POOL_GAUSSIAN, 0.0)])
+def test_no_input_point_reads_nothing(mode, want):
+    """Every neighbour is a pad token and there is no input 0 to read in its place: the kernels that
+    look at the index first take it."""
+    x, y = torch.zeros(1, device="cuda"), torch.full((2, 3, 20), 5.0, device="cuda")
+    nbr = torch.zeros(20, 4, dtype=torch.int32, device="cuda")
+    w = torch.ones(20, 4, device="cuda")
+    a = _lib.KnnPoolArgs()
+    a.x, a.x_dtype, a.y, a.y_dtype = x.data_ptr(), _lib.F32, y.data_ptr(), _lib.F32
+    a.batch, a.channels, a.n_in, a.n_out, a.k = 2, 3, 0, 20, 4
+    a.x_stride[:], a.y_stride[:] = [0, 0, 1], [60, 20, 1]
+    a.nbr, a.weights, a.mode = nbr.data_ptr(), w.data_ptr(), mode
+    _lib.check(_lib.load().fovi_knnpool_fwd(a, _lib.stream_handle(y.device)), "fovi_knnpool_fwd")
+    assert torch.equal(y.nan_to_num(7.0), torch.full_like(y, want).nan_to_num(7.0))
