@@ -390,6 +390,9 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
         self._direct_tables = tiles
         self._packed = {}
         self._img = _ImageRows(slot_ptr, nbr_sorted)
+        self._few_lists = None
+        if self.in_channels <= 8 and slot_ptr.numel():
+            self._few_channel_lists()            # what its weight gradient's choice needs
         order = None
         if tiles is not None:
             order = T.stream_slot_order(T.slot_stream_units(tiles), ahead=T.wide_tiles_of(tiles))
@@ -1047,7 +1050,7 @@ class KNNConvLayer(nn.Module, KNNBaseLayer):
     def _few_channel_lists(self):
         """``(rounds, entries)``: the mean neighbour count of the fullest slot of a block of
         ``32 // c_in`` slots, for the block where it is largest, and the mean list length of a
-        point (from about 256 points, once)."""
+        point (from about 256 points, once, when the tables are built)."""
         if self._few_lists is None:
             ptr = self.slot_ptr.cpu() if self._img is None else self._img.slot_ptr
             cnt = (ptr[::max(1, len(ptr) // 256)] & 0xFFFF).to(torch.float32)

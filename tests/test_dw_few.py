@@ -129,6 +129,7 @@ def test_dw_few_is_taken_where_it_pays():
         assert pays == [False, False, True]
     small = _layer(8, 4, 9, 3, 32, None, device="cpu")          # below the host's own time
     assert small._dw_few_pays(torch.zeros(1, 3, small.in_coords.shape[0]))
+    assert small._few_lists is not None and _layer(8, 4, 9, 9, 32, None, device="cpu")._few_lists is None
     eight = _layer(48, 24, 49, 8, 96, 14, device="cpu")         # channels-last bf16: the pair lists
     rows = lambda b: torch.zeros(b, eight.in_coords.shape[0], 8, dtype=torch.bfloat16).transpose(1, 2)
     assert not eight._dw_few_pays(rows(1)) and eight._dw_few_pays(rows(128))
